@@ -773,7 +773,9 @@ def swept_phasor_program(cfg: SweptPhasorConfig, optimizer: bool = True) -> Prog
     p.add(R.K_ACCUM_TABLE, [time, T], [step, 0.0, 1.0, 0.0, 1.0], flags=R.OP_STATIC, label="time",
           dispatch="static singleThreaded")
     n = float(T * E)
-    p.add(R.K_SWEPT_PHASOR, [slope, time, reset, -1, gup, lossp, E, T, int(cfg.smooth)], [cfg.sr, cfg.base, cfg.target],
+    # the increments' tape lives in dfreq, which the scan writes afterwards
+    p.add(R.K_SWEPT_PHASOR, [slope, time, reset, -1, gup, lossp, E, T, int(cfg.smooth), dfreq, 1],
+          [cfg.sr, cfg.base, cfg.target],
           label="swept_phasor", dispatch=f"fixedWithFrameLoop({E})", bytes=n * f4 + T * 2 * f4, flops=n * 10.0,
           bound="valu")
     p.add(R.K_COLSUM, [lossp, loss, E, 1, 1, ws_col], label="loss_sum", dispatch="chunkPartialsReduceToCell",

@@ -353,7 +353,9 @@ enum dgen_hip_kernel {
    * phase)) against target: loss partials per lane and the upstream gradient.
    * arg: [0]=slope ([E]) [1]=time ([T]) [2]=reset ([T]) or -1 [3]=phase
    *      ([T][E]) or -1 [4]=upstream ([T][E]) [5]=loss partials ([E]) [6]=E
-   *      [7]=T [8]=smooth (0/1)
+   *      [7]=T [8]=smooth (0/1) [9]=scratch ([T][E], 16-byte aligned) when [10]=1
+   *      (the increments are formed ahead of the phase chain; its contents are
+   *      not defined afterwards)
    * farg: [0]=sample rate [1]=base frequency [2]=target */
   DGEN_HIP_K_SWEPT_PHASOR = 32,
 

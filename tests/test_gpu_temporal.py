@@ -65,6 +65,39 @@ def test_scan_matches_oracle(gpu, E, T):
             assert np.all(got[rs > 0] == 0.0)  # a reset frame discards its increment
 
 
+@pytest.mark.parametrize("E,T", [(1, 4), (3, 31), (64, 32), (65, 67), (70, 68), (256, 131), (5, 132), (130, 1027),
+                                 (64, 6 * 32), (2, 4099), (33, 40000)])
+@pytest.mark.parametrize("form", ["rising", "resets", "falling", "inf"])
+def test_swept_phasor_passes_equal_the_one_pass_loop(E, T, form):
+    """With a scratch cell the increments, the phase chain and the loss run as
+    separate passes: phase and upstream gradient are the one-pass loop's bit
+    for bit over every edge of the blocks of 32 and segments of 64 frames,
+    with resets, negative increments and non-finite ones; the loss, fp64 sums
+    in another order rounded to fp32 at the end, to one ulp (1.2e-7)."""
+    rng = np.random.default_rng(E * 7 + T)
+    slope = rng.uniform(-3e4, 3e4, E) if form == "falling" else rng.uniform(100, 3e4, E)
+    time = np.arange(T) / 44100.0
+    if form == "inf":
+        time[rng.integers(0, T, 2)] = [np.inf, 1e35]
+    reset = np.zeros(T) if form in ("rising", "falling") else (rng.random(T) < 0.02).astype(np.float64)
+    got = {}
+    for scratch in (0, 1):
+        p = Program(max_frames=T)
+        c = {n: p.alloc(n, k) for n, k in (("slope", E), ("time", T), ("reset", T), ("phase", T * E), ("g", T * E),
+                                           ("loss", E), ("scratch", T * E))}
+        p.add(R.K_SWEPT_PHASOR, [c["slope"], c["time"], c["reset"], c["phase"], c["g"], c["loss"], E, T, 1,
+                                 c["scratch"], scratch], [44100.0, -20.0 if form == "falling" else 80.0, 0.08])
+        with R.HIPLazyRuntime(p) as rt:
+            for n, a in (("slope", slope), ("time", time), ("reset", reset)):
+                rt.write(n, a)
+            for _ in range(2):
+                rt.runNoCopy()
+            got[scratch] = [rt.read(n) for n in ("phase", "g", "loss")]
+    for a, b in zip(got[0][:2], got[1][:2]):
+        np.testing.assert_array_equal(a, b)
+    np.testing.assert_allclose(got[1][2], got[0][2], rtol=1.2e-7)
+
+
 @pytest.mark.parametrize("reset_from", [-1, 40000])
 def test_swept_phasor_gradient(gpu, reset_from):
     cfg = SweptPhasorConfig(reset_from=reset_from)
