@@ -101,10 +101,11 @@ __device__ __forceinline__ float svf_step(const SvfK& K, float ks, float x, floa
   const float s2 = sat_div<SAT>(c2, ks);
   const float v3 = x - s2;
   const float v1 = K.a1 * s1 + K.a2 * v3;
-  const float ic1 = 2.0f * v1 - s1;
+  // (doubling is exact, so the fma rounds as the product and difference do)
+  const float ic1 = __builtin_fmaf(2.0f, v1, -s1);
   const float v1p = (ic1 + s1) * 0.5f;
   const float v2 = s2 + K.g * v1p;
-  const float ic2 = 2.0f * v2 - s2;
+  const float ic2 = __builtin_fmaf(2.0f, v2, -s2);
   c1 = ic1;
   c2 = ic2;
   return (ic2 + s2) * 0.5f;
@@ -278,13 +279,15 @@ __global__ __launch_bounds__(kThreads) void k_svf_fwd(const float* __restrict__ 
 // the loop's dependency chain).  One load per frame: the sequential loop is
 // bound by its outstanding memory operations, not by arithmetic.
 __global__ __launch_bounds__(kThreads) void k_svf_coef(Ctl ctl, const float* __restrict__ prm,
-                                                       float* __restrict__ tape, int B, int T, int L, float sr) {
-  Lane l;
-  if (!lane_chunk(prm, B, T, L, sr, false, l)) return;
-  for (int n = l.n0; n < l.n1; ++n) {
-    const SvfK K = svf_coef(raw_cutoff(l.base, ctl.m ? ctl.m[n] : 1.0f, ctl.env ? ctl.env[n] : 0.0f, ctl), l.kd,
-                            sr, l.rsr);
-    tape[(size_t)n * B + l.k] = K.g;
+                                                       float* __restrict__ tape, int B, int T, float sr) {
+  const int k = blockIdx.y * kThreads + threadIdx.x;
+  if (k >= B) return;
+  const float base = prm[k], kd = 1.0f / prm[B + k], rsr = rcp_rn(sr);
+  // frames blockIdx.x, + gridDim.x, ...: the tangents are independent, so
+  // short threads in many waves hide their latency
+  for (int n = blockIdx.x; n < T; n += gridDim.x) {
+    const SvfK K = svf_coef(raw_cutoff(base, ctl.m ? ctl.m[n] : 1.0f, ctl.env ? ctl.env[n] : 0.0f, ctl), kd, sr, rsr);
+    tape[(size_t)n * B + k] = K.g;
   }
 }
 
@@ -449,6 +452,218 @@ __global__ __launch_bounds__(64) void k_svf_seq_tiled(const float* __restrict__ 
   if (state) {
     state[k] = c1;
     state[B + k] = c2;
+  }
+}
+
+// ---- saturating forward, parallel in time ---------------------------------
+// The filter forgets: two runs of the recurrence on the same input reach the
+// same fp32 state, to the bit, some frames after they start apart (from zero
+// state: 240 frames for the median lane of SvfConfig's ranges, 700-1250 for
+// nine in ten, 4000-7600 for the most resonant lane with hardly any
+// saturation).  So spans of frames run side by side and a span is known to be
+// right once the state it started from equals, bit for bit, the state the
+// span before it ends in, back to span 0:
+//   k_svf_spec<true>   every span from zero state kSpecWarm frames ahead of it
+//   k_svf_spec<false>  again, the spans whose start differs from the end of
+//                      the span before, from that end; several passes, each
+//                      extending what a span has seen by one span.  Lanes and
+//                      waves with nothing to do leave at once
+//   k_svf_repair       per lane, in order: whatever still differs re-run from
+//                      the end before it, until the states meet again
+// What is left in y, the cells and the loss partials is what k_svf_seq
+// leaves, bit for bit, whatever the input: a lane that never forgets (NaN, or
+// silence after a resonant note, where states shrink together) costs
+// k_svf_repair the sequential loop's time.
+// The time is that of the passes' dependent frames, ~110 ns a frame and wave
+// (~40 instructions, three of them reciprocals, 16 of them one after the
+// other), where the sequential loop took 148 ns for each of all T.  256 lanes
+// x 65536 frames: 9.66 ms for the loop; 0.51 ms here (coefficients 33 us,
+// first pass 91, twelve more at 5 to 60, repair 12).
+// States: start[c][2][B] and, in turn, end0/end1[c][2][B], c a span.
+constexpr int kSpecWarm = 256;  // frames run ahead of a span's first pass
+constexpr int kSpecSpan = 512;  // smallest span
+constexpr int kSpecReach = 6144;  // frames the repeated passes cover
+constexpr int kSpecG = 16;      // frames per prefetch group
+
+// Rows of an array [..][B] from one frame on, as a raw buffer: a row is a
+// uniform byte offset, a lane's column the per-lane one, so a row's six
+// accesses share one scalar add and need no per-lane address.
+using Rows = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ Rows rows_at(const float* p, size_t row, int rows, int B) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p) + row * B, 0, rows * B * (int)sizeof(float),
+                                           0x00020000);
+}
+__device__ __forceinline__ float row_load(Rows r, int col, int row) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, col, row, 0));
+}
+__device__ __forceinline__ void row_store(float v, Rows r, int col, int row) {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, col, row, 0);
+}
+
+// Frames [n0, n1) of 64 lanes from (c1, c2): the recurrence with the tape's
+// coefficients; OUT: y and, with LOSS, the cells and the loss partials of
+// L-frame chunks (n0 a multiple of L, L of kSpecG).  Loads run one group
+// ahead; nothing in a frame branches.
+template <bool OUT, bool LOSS>
+__device__ __forceinline__ void svf_span(const float* __restrict__ x, const float* __restrict__ tape, float kd,
+                                         float ks, float* __restrict__ y, float* __restrict__ cells,
+                                         const float* __restrict__ tgt, float* __restrict__ lossp, int B, int T, int L,
+                                         int k, int n0, int n1, float& c1, float& c2) {
+  const int cnt = n1 - n0;
+  if (cnt <= 0) return;
+  constexpr bool T3 = OUT && LOSS;
+  const Rows rx = rows_at(x, n0, cnt, B), rg = rows_at(tape, n0, cnt, B);
+  const Rows rt = T3 ? rows_at(tgt, n0, cnt, B) : rx, ry = OUT ? rows_at(y, n0, cnt, B) : rx;
+  const Rows ra = T3 ? rows_at(cells, n0, cnt, B) : rx, rb = T3 ? rows_at(cells, (size_t)T + n0, cnt, B) : rx;
+  const int col = k * (int)sizeof(float), pitch = B * (int)sizeof(float);
+  float cx[kSpecG], cg[kSpecG], ct[kSpecG];
+  // (rows past the end read as 0)
+  auto load = [&](int i, float (&vx)[kSpecG], float (&vg)[kSpecG], float (&vt)[kSpecG]) {
+#pragma unroll
+    for (int j = 0; j < kSpecG; ++j) {
+      const int r = (i + j) * pitch;
+      vx[j] = row_load(rx, col, r);
+      vg[j] = row_load(rg, col, r);
+      if constexpr (T3) vt[j] = row_load(rt, col, r);
+    }
+  };
+  float ls = 0.0f;
+  auto frame = [&](int i, float xv, float g, float t) {
+    SvfK K;
+    K.g = g;
+    K.Q = 1.0f + K.g * (K.g + kd);
+    K.a1 = rcp_rn(K.Q);
+    K.a2 = K.g * K.a1;
+    const int r = i * pitch;
+    if constexpr (T3) {
+      row_store(c1, ra, col, r);
+      row_store(c2, rb, col, r);
+    }
+    const float out = svf_step<true>(K, ks, xv, c1, c2);
+    if constexpr (OUT) row_store(out, ry, col, r);
+    if constexpr (T3) {
+      const float d = out - t;
+      ls += d * d;
+    }
+  };
+  auto flush = [&](int i) {
+    if constexpr (T3) {
+      lossp[(size_t)((n0 + i - 1) / L) * B + k] = ls;
+      ls = 0.0f;
+    }
+  };
+  int i = 0, left = L;  // frames to the end of the loss chunk
+  auto group = [&](const float (&vx)[kSpecG], const float (&vg)[kSpecG], const float (&vt)[kSpecG]) {
+#pragma unroll
+    for (int j = 0; j < kSpecG; ++j) frame(i + j, vx[j], vg[j], T3 ? vt[j] : 0.0f);
+    i += kSpecG;
+    left -= kSpecG;
+    if (left == 0) {
+      flush(i);
+      left = L;
+    }
+  };
+  load(0, cx, cg, ct);
+  float nx[kSpecG], ng[kSpecG], nt[kSpecG];
+  while (i + 2 * kSpecG <= cnt) {
+    load(i + kSpecG, nx, ng, nt);
+    __builtin_amdgcn_sched_barrier(0);
+    group(cx, cg, ct);
+    load(i + kSpecG, cx, cg, ct);
+    __builtin_amdgcn_sched_barrier(0);
+    group(nx, ng, nt);
+  }
+  if (i + kSpecG <= cnt) {
+    load(i + kSpecG, nx, ng, nt);
+    group(cx, cg, ct);
+#pragma unroll
+    for (int j = 0; j < kSpecG; ++j) {
+      cx[j] = nx[j];
+      cg[j] = ng[j];
+      if constexpr (T3) ct[j] = nt[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kSpecG; ++j)
+    if (i + j < cnt) frame(i + j, cx[j], cg[j], T3 ? ct[j] : 0.0f);
+  if (left < L || i < cnt) flush(cnt);
+}
+
+struct SpecArgs {
+  const float* x;
+  const float* prm;
+  const float* tape;
+  float* y;
+  float* cells;
+  const float* tgt;
+  float* lossp;
+  float* start;      // [C][2][B]
+  int B, T, L, span, C;
+};
+
+__device__ __forceinline__ bool same_bits(float a, float b) {
+  return __builtin_bit_cast(uint32_t, a) == __builtin_bit_cast(uint32_t, b);
+}
+
+template <bool FIRST, bool LOSS>
+__global__ __launch_bounds__(64) void k_svf_spec(SpecArgs a, const float* __restrict__ ein, float* __restrict__ eout) {
+  const int k = blockIdx.y * 64 + threadIdx.x, c = blockIdx.x, B = a.B;
+  if (k >= B) return;
+  const size_t o1 = (size_t)c * 2 * B + k, o2 = o1 + B;
+  const float kd = 1.0f / a.prm[B + k], ks = a.prm[2 * B + k];
+  const int n0 = c * a.span, n1 = min(a.T, n0 + a.span);
+  float c1 = 0.0f, c2 = 0.0f;
+  if constexpr (FIRST) {
+    svf_span<false, false>(a.x, a.tape, kd, ks, nullptr, nullptr, nullptr, nullptr, B, a.T, a.L, k,
+                           max(0, n0 - kSpecWarm), n0, c1, c2);
+  } else {
+    if (c > 0) {
+      c1 = ein[o1 - 2 * (size_t)B];
+      c2 = ein[o2 - 2 * (size_t)B];
+    }
+    if (c == 0 || (same_bits(c1, a.start[o1]) && same_bits(c2, a.start[o2]))) {
+      eout[o1] = ein[o1];
+      eout[o2] = ein[o2];
+      return;
+    }
+  }
+  a.start[o1] = c1;
+  a.start[o2] = c2;
+  svf_span<true, LOSS>(a.x, a.tape, kd, ks, a.y, a.cells, a.tgt, a.lossp, B, a.T, a.L, k, n0, n1, c1, c2);
+  eout[o1] = c1;
+  eout[o2] = c2;
+}
+
+// Workgroup: 64 lanes; its waves look for spans that differ, then the first
+// wave repairs them in order.
+constexpr int kRepairWaves = 8;
+template <bool LOSS>
+__global__ __launch_bounds__(64 * kRepairWaves) void k_svf_repair(SpecArgs a, const float* __restrict__ end) {
+  __shared__ int s_bad[kRepairWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, B = a.B;
+  const int kk = blockIdx.x * 64 + lane, k = min(kk, B - 1);
+  int bad = a.C;  // first span that does not start where the one before ends
+  for (int c = 1 + wave; c < a.C; c += kRepairWaves) {
+    const size_t o = (size_t)c * 2 * B + k, e = o - 2 * (size_t)B;
+    if (!same_bits(a.start[o], end[e]) || !same_bits(a.start[o + B], end[e + B])) bad = min(bad, c);
+  }
+  s_bad[wave][lane] = kk < B ? bad : a.C;
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int w = 0; w < kRepairWaves; ++w) bad = min(bad, s_bad[w][lane]);
+  if (kk >= B || bad >= a.C) return;
+  const float kd = 1.0f / a.prm[B + k], ks = a.prm[2 * B + k];
+  size_t o = (size_t)bad * 2 * B + k;
+  float c1 = end[o - 2 * (size_t)B], c2 = end[o - (size_t)B];
+  for (int c = bad; c < a.C; ++c, o += 2 * (size_t)B) {
+    if (same_bits(c1, a.start[o]) && same_bits(c2, a.start[o + B])) {
+      c1 = end[o];
+      c2 = end[o + B];
+    } else {
+      const int n0 = c * a.span, n1 = min(a.T, n0 + a.span);
+      svf_span<true, LOSS>(a.x, a.tape, kd, ks, a.y, a.cells, a.tgt, a.lossp, B, a.T, a.L, k, n0, n1, c1, c2);
+    }
   }
 }
 
@@ -686,6 +901,7 @@ int launch_svf_seq(const Launch& L, const dgen_hip_op& op) {
   // arg: [0]=x [1]=mod [2]=env [3]=params ([3][B]) [4]=state ([2][B]) or -1 [5]=y [6]=cells or -1
   //      [7]=target or -1 [8]=loss partials ([C][B]) or -1 [9]=B [10]=T [11]=L [12]=sanitize
   //      [13]=coefficient tape ([T][B]) or -1
+  //      [14]=span states (6*C*B floats, C = ceil(T/L)) when [15]=1
   // As DGEN_HIP_K_STREAM_SVF: state required, no cells or loss, and a run
   // processes the first frame_count frames.
   const int64_t x = op.arg[0], prm = op.arg[3], st = op.arg[4], y = op.arg[5], cl = op.arg[6], tgt = op.arg[7],
@@ -712,6 +928,12 @@ int launch_svf_seq(const Launch& L, const dgen_hip_op& op) {
     DGEN_CHECK_CELL(L, lossp, s.C * s.B, "svf_seq.loss_partials");
   }
   if (tape >= 0) DGEN_CHECK_CELL(L, tape, s.B * s.T, "svf_seq.coefficient_tape");
+  const bool spec = op.arg[15] == 1;
+  DGEN_REQUIRE(op.arg[15] == 0 || spec, "svf_seq: arg[15] %lld (0, or 1 with span states)", (long long)op.arg[15]);
+  if (spec) {
+    DGEN_REQUIRE(tape >= 0 && st < 0 && !stream, "svf_seq: spans need the coefficient tape and no state cell");
+    DGEN_CHECK_CELL(L, op.arg[14], 6 * s.C * s.B, "svf_seq.span_states");
+  }
   if (L.dry) return 0;
   const dim3 grid((unsigned)((s.B + kSeqThreads - 1) / kSeqThreads));
   float* sp = st >= 0 ? cell(L, st) : nullptr;
@@ -719,12 +941,54 @@ int launch_svf_seq(const Launch& L, const dgen_hip_op& op) {
   const int reset = stream && L.reset ? 1 : 0, san = op.arg[12] ? 1 : 0;
   float* tp = tape >= 0 ? cell(L, tape) : nullptr;
   if (tp) {
-    hipLaunchKernelGGL(k_svf_coef, svf_grid(s), dim3(kThreads), 0, L.stream, ctl, cell(L, prm), tp, (int)s.B,
-                       (int)s.T, (int)s.L, sr);
+    hipLaunchKernelGGL(k_svf_coef, dim3((unsigned)std::min<int64_t>(s.T, 1 << 15), (unsigned)((s.B + kThreads - 1) / kThreads)),
+                       dim3(kThreads), 0, L.stream, ctl, cell(L, prm), tp, (int)s.B, (int)s.T, sr);
     DGEN_LAUNCH_CHECK("k_svf_coef");
   }
   float* tg = tgt >= 0 ? cell(L, tgt) : nullptr;
   float* lp = lossp >= 0 ? cell(L, lossp) : nullptr;
+  const int64_t groups = (s.B + 63) / 64;
+  const int64_t per = std::max<int64_t>((kSpecSpan + s.L - 1) / s.L, groups * s.C / (4 * L.cu_count));
+  // the spans keep the training step's outputs (all or y alone), take whole
+  // prefetch groups to a loss chunk and address a span's rows in 31 bits
+  if (spec && s.C > 1 && !san && (tgt >= 0) == (cl >= 0) && s.L % kSpecG == 0 && per * s.L * s.B < (1ll << 28)) {
+    // spans of whole loss chunks, at least kSpecSpan frames, longer where the
+    // lanes alone give every SIMD a wave: a pass then still fills the chip
+    // once and each one extends what a span has seen by more
+    SpecArgs a{};
+    a.x = cell(L, x);
+    a.prm = cell(L, prm);
+    a.tape = tp;
+    a.y = cell(L, y);
+    a.cells = cp;
+    a.tgt = tg;
+    a.lossp = lp;
+    a.B = (int)s.B;
+    a.T = (int)T;
+    a.L = (int)s.L;
+    a.span = (int)(per * s.L);
+    a.C = (int)((T + a.span - 1) / a.span);
+    float* e[2];
+    a.start = cell(L, op.arg[14]);
+    e[0] = a.start + 2 * (size_t)a.C * a.B;
+    e[1] = e[0] + 2 * (size_t)a.C * a.B;
+    const dim3 sg((unsigned)a.C, (unsigned)groups);
+    // passes that cover kSpecReach frames; what forgets more slowly is left to
+    // the repair
+    const int passes = std::min<int>(a.C - 1, (kSpecReach + a.span - 1) / a.span);
+    auto go = [&](auto first, auto again, auto repair) {
+      hipLaunchKernelGGL(first, sg, dim3(64), 0, L.stream, a, nullptr, e[0]);
+      for (int p = 0; p < passes; ++p)
+        hipLaunchKernelGGL(again, sg, dim3(64), 0, L.stream, a, e[p & 1], e[(p + 1) & 1]);
+      hipLaunchKernelGGL(repair, dim3((unsigned)groups), dim3(64 * kRepairWaves), 0, L.stream, a, e[passes & 1]);
+    };
+    if (tgt >= 0)
+      go(k_svf_spec<true, true>, k_svf_spec<false, true>, k_svf_repair<true>);
+    else
+      go(k_svf_spec<true, false>, k_svf_spec<false, false>, k_svf_repair<false>);
+    DGEN_LAUNCH_CHECK("k_svf_spec");
+    return 0;
+  }
   if (tgt >= 0 && tp && cp && !stream && s.B % 64 == 0 && T % kTileF == 0 && s.L % kTileF == 0) {
     // the training forward through LDS tiles (the same arithmetic)
     hipLaunchKernelGGL(k_svf_seq_tiled, dim3((unsigned)(s.B / 64)), dim3(64), 0, L.stream, cell(L, x), cell(L, prm),

@@ -630,8 +630,10 @@ def svf_program(cfg: SvfConfig, train: bool = True, optimizer: bool = True, satu
     # per lane-frame: coefficients (clip, div, tan, 1/Q, 4 mul/add) ~ 30 flops, one SVF frame 12
     if sat:
         tape = p.alloc("coef_tape", T * B)
-        p.add(R.K_SVF_SEQ, [x, mod, env, prm, -1, y, cells, tgt, lossp, B, T, L, 0, tape], sr, label="svf_seq",
-              dispatch=f"coefficient tape + fixedWithFrameLoop({B})",
+        # the span states live in the adjoint summaries, which are written later
+        spans = asumm if train else p.alloc("span_states", 6 * C * B)
+        p.add(R.K_SVF_SEQ, [x, mod, env, prm, -1, y, cells, tgt, lossp, B, T, L, 0, tape, spans, 1], sr,
+              label="svf_seq", dispatch=f"coefficient tape + spans side by side ({B})",
               bytes=n * f4 * ((5 if train else 2) + 2) + ctl_b, flops=n * (30 + 18), bound="valu")
     else:
         summ = p.alloc("summary", 12 * C * B)  # fp64

@@ -392,6 +392,10 @@ enum dgen_hip_kernel {
    *      [10]=T [11]=L [12]=sanitize (non-finite out stores -> 0)
    *      [13]=coefficient tape ([T][B]: g, filled by the call before the
    *      sequential loop reads it) or -1 (evaluated in the loop)
+   *      [14]=span states (6*C*B floats, C = ceil(T/L)) when [15]=1: spans of
+   *      frames run side by side from speculated states, repeated until each
+   *      starts bit for bit where the one before ends (the same results; needs
+   *      the tape and no state cell)
    * With a target, cells and a tape, B a multiple of 64 and T and L of 32,
    * the loop runs on 32-frame LDS tiles (the same results). */
   DGEN_HIP_K_SVF_SEQ = 35,

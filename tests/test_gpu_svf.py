@@ -9,7 +9,8 @@ import pytest
 
 import oracle as O
 from dgen_hip import SvfConfig
-from dgen_hip.programs import SvfSession, stream_svf_program
+from dgen_hip import runtime as R
+from dgen_hip.programs import SvfSession, stream_svf_program, svf_program
 from dgen_hip.runtime import HIPLazyRuntime
 
 
@@ -192,3 +193,41 @@ def test_saturating_training_loss_covers_a_ragged_last_chunk(B, T, chunk):
     print(f"loss HIP {loss:.8e}, fp64 oracle {l64:.8e}, fp32 oracle {l32:.8e}")
     assert abs(loss - l64) <= 2.0 * abs(l32 - l64) + 1e-5 * abs(l64)
     assert np.linalg.norm(g - g64) <= 1e-4 * np.linalg.norm(g64)
+
+
+@pytest.mark.parametrize("B,T,chunk,signal", [(1, 257, 256, "noise"), (3, 5000, 256, "noise"), (64, 4096, 256, "noise"),
+                                              (70, 3001, 7, "noise"), (256, 20000, 512, "noise"),
+                                              (300, 6145, 96, "noise"), (66, 16384, 256, "click"),
+                                              (5, 12000, 256, "nan"), (64, 9000, 100, "inf")])
+def test_saturating_spans_equal_the_frame_loop(B, T, chunk, signal):
+    """The saturating forward as spans run side by side leaves y, the cells
+    and the loss partials of the per-lane frame loop bit for bit: ragged lane
+    groups, spans and chunks; a click after which the states shrink together
+    and never meet (the repair's part); non-finite input from some frame on."""
+    cfg = SvfConfig(B=B, T=T, saturating=True)
+    rng = np.random.default_rng(B + T)
+    x = rng.uniform(-1, 1, (T, B)).astype(np.float32)
+    if signal == "click":
+        x[1000:] = 0.0
+    elif signal in ("nan", "inf"):
+        x[T // 3, ::2] = np.nan if signal == "nan" else np.inf
+    tgt = rng.uniform(-1, 1, (T, B)).astype(np.float32)
+    prm = cfg.params().reshape(3, B).copy()
+    prm[2, ::3] *= 0.01  # lanes that hardly saturate forget most slowly
+    print(f"case B={B} T={T} chunk={chunk} {signal}", flush=True)
+    got = {}
+    for spans in (0, 1):
+        prog = svf_program(cfg, optimizer=False, chunk=chunk)
+        assert prog.ops[0].kernel == R.K_SVF_SEQ and prog.ops[0].arg[15] == 1
+        prog.ops[0].arg[15] = spans
+        with HIPLazyRuntime(prog) as rt:
+            for name, a in (("x", x), ("target", tgt), ("mod", cfg.modulation()), ("env", cfg.envelope()),
+                            ("params", prm)):
+                rt.write(name, a)
+            for _ in range(2):
+                rt.runNoCopy()
+            got[spans] = [rt.read(n) for n in ("y", "cells", "loss_partials")]
+    for a, b in zip(got[0], got[1]):
+        bits = [np.where(np.isnan(v), 0, v.view(np.uint32)) for v in (a, b)]  # a NaN's sign is not defined
+        np.testing.assert_array_equal(np.isnan(a), np.isnan(b))
+        np.testing.assert_array_equal(*bits)
