@@ -27,6 +27,7 @@ SPLITK_ROWS_HEADS = 256  # the heads' weight gradient has one 128-wide column ti
 MSS_TILE = 4096     # output samples per spectral-loss workgroup
 BQ_CHUNK = 512      # frames per biquad scan chunk (512 measured fastest of 128..1024)
 SVF_CHUNK = 256     # frames per SVF scan chunk
+SCAN_WAVES = 2048   # waves (64 lanes x one chunk) a filter scan's passes should have: two per SIMD
 STFT_TILE = 8192    # output samples per STFT forward workgroup
 MEM_STEPS = 16      # membrane frames per time-blocked launch
 MEM_TILE = 32       # membrane cells per workgroup tile side
@@ -442,6 +443,22 @@ class HarmonicSession:
 
 
 # ------------------------------------------------------------------ config 4
+def _scan_chunk(B: int, T: int, chunk: int) -> int:
+    """Frames per chunk of a filter bank's scans: `chunk`, halved (to no less
+    than 32, in whole thirty-twos) while the lanes and chunks make fewer than
+    SCAN_WAVES waves.  A pass lasts as long as one chunk's frames in sequence
+    (~0.25 us each), so few lanes or a short signal want shorter chunks; with
+    the chip full, shorter ones only add chunk maps to the carry.  Steps
+    measured: biquad 12 lanes x 8192 frames 488 us at 512, 134 at 32, 137 at
+    16; linear SVF 70 x 30001 368 us at 256, 216 at 64, 197 at 32, 236 at 16;
+    saturating SVF 256 x 65536 814 us at 256, 755 at 128, 765 at 64; biquad 256
+    x 2^18 605 us at 512 (kept), 624 at 256, 678 at 128."""
+    L, groups = chunk, (B + 63) // 64
+    while L % 64 == 0 and groups * ((T + L - 1) // L) < SCAN_WAVES:
+        L //= 2
+    return L
+
+
 def _colsum_ws(rows: int, cols: int) -> int:
     return max(1, min(256, rows // 32)) * cols
 
@@ -461,6 +478,7 @@ def biquad_program(cfg: BiquadConfig, train: bool = True, optimizer: bool = True
     B, T, L = cfg.B, cfg.T, int(chunk)
     if L <= 0:
         raise ValueError("chunk length must be positive")
+    L = _scan_chunk(B, T, L)
     C = (T + L - 1) // L
     f4 = 4.0
     p = Program(max_frames=T)
@@ -609,6 +627,7 @@ def svf_program(cfg: SvfConfig, train: bool = True, optimizer: bool = True, satu
     if L <= 0:
         raise ValueError("chunk length must be positive")
     P = 3 if sat else 2
+    L = _scan_chunk(B, T, L)
     C = (T + L - 1) // L
     f4 = 4.0
     n = float(T * B)
