@@ -108,6 +108,7 @@ struct dgen_hip_ctx {
   uint64_t floats = 0;
   uint32_t max_frames = 0;
   std::vector<dgen_hip_op> ops;
+  bool has_side = false;  // any op runs on the side stream
   bool configured = false;
   // graph replay of the per-run schedule (dgen_hip_set_graphs)
   bool use_graphs = false;
@@ -174,14 +175,18 @@ static void release_arena(dgen_hip_ctx* c) {
 
 // Enqueue ops [0, n) that match `static_pass`; optional per-op event timing.
 static int enqueue(dgen_hip_ctx* c, uint32_t frames, bool static_pass, std::vector<hipEvent_t>* evs) {
-  DGEN_HIP_TRY(hipEventRecord(c->ev_start, c->s0));
-  DGEN_HIP_TRY(hipStreamWaitEvent(c->s1, c->ev_start, 0));
+  // (a schedule without side ops leaves the second stream alone: a run of two
+  // kernels takes 17 us to its end so, 32 us with the record and the wait)
+  if (c->has_side) {
+    DGEN_HIP_TRY(hipEventRecord(c->ev_start, c->s0));
+    DGEN_HIP_TRY(hipStreamWaitEvent(c->s1, c->ev_start, 0));
+  }
   bool side_used = false;
   for (size_t i = 0; i < c->ops.size(); ++i) {
     const dgen_hip_op& op = c->ops[i];
     bool is_static = (op.flags & DGEN_HIP_OP_STATIC) != 0;
     if (is_static != static_pass) continue;
-    if (op.flags & DGEN_HIP_OP_JOIN) {
+    if ((op.flags & DGEN_HIP_OP_JOIN) && c->has_side) {
       DGEN_HIP_TRY(hipEventRecord(c->ev_side, c->s1));
       DGEN_HIP_TRY(hipStreamWaitEvent(c->s0, c->ev_side, 0));
     }
@@ -342,6 +347,8 @@ int dgen_hip_configure(dgen_hip_ctx* c, const dgen_hip_op* ops, uint32_t n_ops, 
   memset(c->h_arena, 0, bytes);
   DGEN_HIP_TRY(hipMemsetAsync(c->d_arena, 0, bytes, c->s0));
   c->ops.assign(ops, ops + n_ops);
+  c->has_side = false;
+  for (const auto& op : c->ops) c->has_side |= (op.flags & DGEN_HIP_OP_SIDE) != 0;
   c->max_frames = max_frames;
   c->configured = true;
   return run_static(c);
@@ -481,27 +488,42 @@ int dgen_hip_set_graphs(dgen_hip_ctx* c, int enable) {
   return 0;
 }
 
-// Wait for both streams (no output download).
+// Wait for the context's streams (no output download).
 static int sync_streams(dgen_hip_ctx* c) {
   int rc = set_device(c);
   if (rc) return rc;
   DGEN_HIP_TRY(hipStreamSynchronize(c->s0));
-  DGEN_HIP_TRY(hipStreamSynchronize(c->s1));
+  if (c->has_side) DGEN_HIP_TRY(hipStreamSynchronize(c->s1));
+  return 0;
+}
+
+// Queue a copy behind stream 0's work (a run's side work is joined into it);
+// the caller waits for the streams before it uses or rewrites the mirror.
+static int queue_to_host(dgen_hip_ctx* c, uint64_t off, uint64_t n) {
+  if (!n) return 0;
+  DGEN_HIP_TRY(hipMemcpyAsync(c->h_arena + off, c->d_arena + off, n * sizeof(float), hipMemcpyDeviceToHost, c->s0));
+  return 0;
+}
+static int queue_to_device(dgen_hip_ctx* c, uint64_t off, uint64_t n) {
+  if (!n) return 0;
+  DGEN_HIP_TRY(hipMemcpyAsync(c->d_arena + off, c->h_arena + off, n * sizeof(float), hipMemcpyHostToDevice, c->s0));
   return 0;
 }
 
 int dgen_hip_sync(dgen_hip_ctx* c) {
   if (!c) return fail(DGEN_HIP_E_INVALID, "sync: null context");
-  int rc = sync_streams(c);
-  if (rc) return rc;
   // the declared outputs of a dgen_hip_run_async become host-visible here, as
   // the reference's shared-storage outputs buffer is after run()
-  // (MetalRuntime.swift:232, 334-337)
+  // (MetalRuntime.swift:232, 334-337); their copy is queued behind the run,
+  // so one wait covers both
+  int rc = set_device(c), rc_copy = 0;
+  if (rc) return rc;
   if (c->outputs_pending) {
     c->outputs_pending = false;
-    if (c->out_n) return dgen_hip_download(c, c->out_off, c->out_n);
+    rc_copy = queue_to_host(c, c->out_off, c->out_n);
   }
-  return 0;
+  rc = sync_streams(c);
+  return rc ? rc : rc_copy;
 }
 
 int dgen_hip_run(dgen_hip_ctx* c, uint32_t frame_count) {
@@ -619,21 +641,27 @@ int dgen_hip_process_v1(dgen_hip_ctx* c, const float* const* inputs, float* cons
       const uint32_t st = c->in_stride[i];
       for (uint32_t f = 0; f < frame_count; ++f) dst[(size_t)f * st] = inputs[i][f];
     }
-    if ((rc = dgen_hip_upload(c, lo, hi - lo))) return rc;
+    if ((rc = queue_to_device(c, lo, hi - lo))) {
+      (void)sync_streams(c);
+      return rc;
+    }
   }
-  // the run, eagerly enqueued, at the call's host rate and reset flag
+  // the run, eagerly enqueued behind the inputs' copy, at the call's host rate and reset flag
   const float saved_sr = c->host_sr;
   c->host_sr = sr;
   c->reset_next = (flags & DGEN_HIP_PROCESS_RESET) != 0;
   rc = enqueue(c, frame_count, false, nullptr);
   c->host_sr = saved_sr;
   c->reset_next = false;
+  // the outputs' copy behind the run: one wait for the call's copies and run
+  uint64_t lo = 0, hi = 0;
+  if (!rc && !c->out_cell.empty()) {
+    port_span(c->out_cell, c->out_stride, frame_count, &lo, &hi);
+    rc = queue_to_host(c, lo, hi - lo);
+  }
   const int rc2 = dgen_hip_sync(c);
   if (rc || rc2) return rc ? rc : rc2;
   if (!c->out_cell.empty()) {
-    uint64_t lo, hi;
-    port_span(c->out_cell, c->out_stride, frame_count, &lo, &hi);
-    if ((rc = dgen_hip_download(c, lo, hi - lo))) return rc;
     for (size_t i = 0; i < c->out_cell.size(); ++i) {
       const float* src = c->h_arena + c->out_cell[i];
       const uint32_t st = c->out_stride[i];

@@ -192,6 +192,12 @@ class KernelTiming:
     gpu_ms: float
 
 
+def _channels(addresses):
+    """A float** of channel addresses."""
+    return ctypes.cast((ctypes.c_void_p * max(1, len(addresses)))(*addresses),
+                       ctypes.POINTER(ctypes.POINTER(ctypes.c_float)))
+
+
 class HIPLazyRuntime:
     """Runtime for one compiled program on one device (LazyRuntime mirror)."""
 
@@ -319,13 +325,15 @@ class HIPLazyRuntime:
     def process(self, inputs, frames: int, sample_rate: float = 0.0, reset: bool = False) -> np.ndarray:
         """One dgen_hip_process_v1 block: inputs [n_in][frames] -> outputs [n_out][frames]."""
         n_in, n_out = self._ports
-        fp = ctypes.POINTER(ctypes.c_float)
         ins = [np.ascontiguousarray(a, np.float32) for a in inputs]
         if len(ins) != n_in or any(a.shape != (frames,) for a in ins):
             raise ValueError(f"process: {n_in} input channels of {frames} frames expected")
         outs = np.zeros((n_out, frames), np.float32)
-        ip = (fp * max(1, n_in))(*[a.ctypes.data_as(fp) for a in ins])
-        op = (fp * max(1, n_out))(*[outs[i].ctypes.data_as(fp) for i in range(n_out)])
+        # channel pointers as plain addresses (a ctypes pointer object per
+        # channel cost ~2 us each)
+        at = outs.__array_interface__["data"][0]
+        ip = _channels([a.__array_interface__["data"][0] for a in ins])
+        op = _channels([at + 4 * frames * i for i in range(n_out)])
         ctxv = CProcessContext(2, ctypes.sizeof(CProcessContext), float(sample_rate), PROCESS_RESET if reset else 0)
         _check(self.L.dgen_hip_process_v1(self._ctx, ip, op, int(frames), ctypes.byref(ctxv)), "dgen_hip_process_v1")
         return outs
