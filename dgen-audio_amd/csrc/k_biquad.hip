@@ -605,42 +605,123 @@ int launch_biquad_bwd(const Launch& L, const dgen_hip_op& op) {
   return 0;
 }
 
-// ---- streaming bank: one thread per lane, history carried between runs ----
-// The reference's per-lane frame loop (StatefulTensorParallelPolicy.swift:
-// 21-74): lane k steps Direct Form I frame by frame in registers from the
-// history cells state[4][B] (x[n-1], x[n-2], y[n-1], y[n-2]) and writes them
-// back, so any split of a run into runs gives the same samples; frames are
-// read and written [frame][lane] (a wave's 64 lanes are 256 contiguous
-// bytes).  Out stores map non-finite values to 0 (CRenderer.swift:1021-1039).
+// ---- streaming bank: history carried between runs --------------------------
+// The per-lane frame loop of the reference's C backend on one block of frames.
+// The state cell ([4][B]: x[n-1], x[n-2], y[n-1], y[n-2]) is read at a run's
+// start and written back, and every frame's arithmetic is the same wherever
+// it lies in a run, so any split of a run into runs gives the same samples.
+// Out stores map non-finite values to 0 (CRenderer.swift:1021-1039).
+//
+// Only y[n] = F[n] - a2[n] y[n-2] - a1[n] y[n-1] is sequential, one dependent
+// fma a frame; the coefficients and the input part F are not.  One thread per
+// lane doing all of it issued ~100 instructions a frame from one wave: 97 us
+// for 16 lanes x 512 frames.  Here a workgroup takes kSbLanes lanes: waves 1-3
+// form F, a1, a2 of the next kSbF frames in LDS (and store the y of the
+// previous ones) while wave 0 steps the current ones: 11 us.  Few lanes per
+// workgroup, because forming one frame's coefficients costs ~20 times a step.
+constexpr int kSbLanes = 8;
+constexpr int kSbF = 96;            // frames per tile: 4 elements per forming thread
+constexpr int kSbLd = kSbF + 4;     // LDS row (16-byte aligned, lanes on different banks)
+constexpr int kSbForm = kThreads - 64;
+static_assert(kSbLanes * kSbF % kSbForm == 0, "whole elements per forming thread");
+
 template <bool MOD>
 __global__ __launch_bounds__(kThreads) void k_stream_bq(const float* __restrict__ x, const float* __restrict__ mod,
                                                         const float* __restrict__ prm, float* __restrict__ state,
                                                         float* __restrict__ y, int B, int T, int reset) {
-  const int k = blockIdx.x * kThreads + threadIdx.x;
-  if (k >= B) return;
-  const float base = prm[k], q = fabsf(prm[B + k]), rq = 1.0f / q;
-  float x1 = 0.f, x2 = 0.f, y1 = 0.f, y2 = 0.f;
-  if (!reset) {
-    x1 = state[k];
-    x2 = state[B + k];
+  __shared__ __align__(16) float sF[2][kSbLanes][kSbLd], s1[2][kSbLanes][kSbLd], s2[2][kSbLanes][kSbLd];
+  __shared__ __align__(16) float sy[2][kSbLanes][kSbLd];
+  const int ntile = (T + kSbF - 1) / kSbF, k0 = blockIdx.x * kSbLanes;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // forming thread j: elements (lane j % kSbLanes, frames j / kSbLanes + i * step)
+  const int j = (int)threadIdx.x - 64, l = threadIdx.x % kSbLanes, k = k0 + l;
+  constexpr int kStep = kSbForm / kSbLanes, kPer = kSbF / kStep;
+  const bool live = k < B;
+  float base = 0.0f, q = 1.0f, rq = 1.0f, h1 = 0.0f, h2 = 0.0f;  // h: x[-1], x[-2]
+  if (live) {
+    base = prm[k];
+    q = fabsf(prm[B + k]);
+    rq = 1.0f / q;
+    if (!reset) {
+      h1 = state[k];
+      h2 = state[B + k];
+    }
+  }
+  auto form = [&](int t) {
+    const int b = t & 1;
+    float x0[kPer], x1[kPer], x2[kPer], m[kPer];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int n = t * kSbF + j / kSbLanes + i * kStep;
+      const bool in = live && n < T;
+      x0[i] = in ? x[(size_t)n * B + k] : 0.0f;
+      x1[i] = in && n >= 1 ? x[(size_t)(n - 1) * B + k] : h1;
+      x2[i] = in && n >= 2 ? x[(size_t)(n - 2) * B + k] : (n == 1 ? h1 : h2);
+      m[i] = MOD && n < T ? mod[n] : 1.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int f = j / kSbLanes + i * kStep;
+      const Coef K = coef(base * m[i], q, rq);
+      sF[b][l][f] = __builtin_fmaf(x0[i], K.b0, __builtin_fmaf(x1[i], K.b1, x2[i] * K.b0));
+      s1[b][l][f] = K.a1;
+      s2[b][l][f] = K.a2;
+    }
+  };
+  auto store = [&](int t) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int f = j / kSbLanes + i * kStep, n = t * kSbF + f;
+      const float v = sy[t & 1][l][f];
+      if (live && n < T) y[(size_t)n * B + k] = isfinite(v) ? v : 0.f;
+    }
+  };
+  float y1 = 0.0f, y2 = 0.0f;  // wave 0, threads below kSbLanes
+  const bool chain = threadIdx.x < kSbLanes && live;
+  if (chain && !reset) {
     y1 = state[2 * B + k];
     y2 = state[3 * B + k];
   }
-  const float* const src[1] = {x};
-  walk_fwd<1, MOD>(src, mod, B, k, 0, T, [&](int n, const float* v, float m) {
-    const Coef K = coef(base * m, q, rq);
-    const float x0 = v[0];
-    const float out = ((x2 * K.b0 + x1 * K.b1) + x0 * K.b0) - (y2 * K.a2 + y1 * K.a1);
-    y[(size_t)n * B + k] = isfinite(out) ? out : 0.f;
-    y2 = y1;
-    y1 = out;
-    x2 = x1;
-    x1 = x0;
-  });
-  state[k] = x1;
-  state[B + k] = x2;
-  state[2 * B + k] = y1;
-  state[3 * B + k] = y2;
+  if (wave > 0) form(0);
+  __syncthreads();
+  for (int t = 0; t < ntile; ++t) {
+    if (wave > 0) {
+      if (t + 1 < ntile) form(t + 1);
+      if (t > 0) store(t - 1);
+    } else if (chain) {
+      const int b = t & 1, nf = min(kSbF, T - t * kSbF);
+      const float4* pF = reinterpret_cast<const float4*>(sF[b][l]);
+      const float4* p1 = reinterpret_cast<const float4*>(s1[b][l]);
+      const float4* p2 = reinterpret_cast<const float4*>(s2[b][l]);
+      float4* py = reinterpret_cast<float4*>(sy[b][l]);
+      auto step = [&](float F, float a1, float a2) {
+        const float o = __builtin_fmaf(-y1, a1, __builtin_fmaf(-y2, a2, F));
+        y2 = y1;
+        y1 = o;
+        return o;
+      };
+      int g = 0;
+#pragma unroll 4
+      for (; g < nf / 4; ++g) {
+        const float4 F = pF[g], a1 = p1[g], a2 = p2[g];
+        float4 o;
+        o.x = step(F.x, a1.x, a2.x);
+        o.y = step(F.y, a1.y, a2.y);
+        o.z = step(F.z, a1.z, a2.z);
+        o.w = step(F.w, a1.w, a2.w);
+        py[g] = o;
+      }
+      for (int f = 4 * g; f < nf; ++f) sy[b][l][f] = step(sF[b][l][f], s1[b][l][f], s2[b][l][f]);
+    }
+    __syncthreads();
+  }
+  if (wave > 0) store(ntile - 1);
+  if (chain) {
+    state[k] = x[(size_t)(T - 1) * B + k];
+    state[B + k] = T >= 2 ? x[(size_t)(T - 2) * B + k] : h1;
+    state[2 * B + k] = y1;
+    state[3 * B + k] = y2;
+  }
 }
 
 int launch_stream_biquad(const Launch& L, const dgen_hip_op& op) {
@@ -657,7 +738,7 @@ int launch_stream_biquad(const Launch& L, const dgen_hip_op& op) {
   DGEN_CHECK_CELL(L, y, B * T, "stream_biquad.y");
   if (L.dry) return 0;
   const int64_t n = std::min<int64_t>(T, L.frames ? (int64_t)L.frames : T);
-  const dim3 grid((unsigned)((B + kThreads - 1) / kThreads));
+  const dim3 grid((unsigned)((B + kSbLanes - 1) / kSbLanes));
   if (mod >= 0)
     hipLaunchKernelGGL(k_stream_bq<true>, grid, dim3(kThreads), 0, L.stream, cell(L, x), cell(L, mod), cell(L, prm),
                        cell(L, st), cell(L, y), (int)B, (int)n, L.reset ? 1 : 0);

@@ -134,3 +134,32 @@ def test_biquad_bank_calls(gpu):
           f"{np.abs(one - ref).max():.3e}")
     assert np.abs(one - ref).max() < 1e-4
     assert e_hip <= 2.0 * e_o32 + 1e-7
+
+
+@pytest.mark.parametrize("B,sizes", [(1, [1, 1, 2, 96, 97]), (7, [95, 96, 3]), (8, [192, 500]), (9, [193, 1, 100]),
+                                     (65, [1000, 7]), (16, [512] * 3)])
+def test_biquad_blocks_over_tile_edges(B, sizes):
+    """Lane groups of 8 and tiles of 96 frames: blocks that end on, before and
+    after a tile give the samples of one call bit for bit, with an infinite
+    input sample stored as 0 while the history keeps it; within twice the fp32
+    oracle's distance of the fp64 oracle."""
+    T = sum(sizes)
+    cfg = BiquadConfig(B=B, T=T)
+    x, mod = cfg.inputs(), cfg.modulation()
+    print(f"streaming biquad bank B={B} blocks {sizes}", flush=True)
+    rt = bq_runtime(cfg)
+    try:
+        one = bq_calls(rt, x, mod, [T])
+        np.testing.assert_array_equal(bq_calls(rt, x, mod, sizes), one)
+        bad = x.copy()
+        bad[T // 2, 0] = np.inf
+        split, whole = bq_calls(rt, bad, mod, sizes), bq_calls(rt, bad, mod, [T])
+        np.testing.assert_array_equal(split, whole)
+        assert np.isfinite(whole).all() and not whole[T // 2:, 0].any()
+        np.testing.assert_array_equal(whole[:T // 2], one[:T // 2])
+    finally:
+        rt.close()
+    p = cfg.params()
+    ref = O.biquad_stream(x, mod, p[:B], p[B:], np.zeros((B, 4), np.float32))
+    ref64 = O.biquad_fwd(x, mod, p[:B].astype(np.float64), p[B:].astype(np.float64), prec="f64")
+    assert np.abs(one - ref64).max() <= 2.0 * np.abs(ref - ref64).max() + 1e-7
