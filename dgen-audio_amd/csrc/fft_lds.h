@@ -195,6 +195,42 @@ struct RegTwiddle {
   }
 };
 
+// HwTwiddle's values for one thread's butterflies, in registers: the same
+// hardware sin/cos and products, evaluated once per kernel instead of in every
+// transform (the inverse's are the conjugates, bit for bit).
+template <int LOGM>
+struct HwRegTwiddle {
+  static constexpr bool kTable = true;
+  static constexpr int M = 1 << LOGM, NP = pass_count(LOGM);
+  template <int R, int NS>
+  static constexpr int nu() { return (M / 8) % NS == 0 ? 1 : 8 / R; }
+  c2 w[NP][4][7];  // [pass][u][r - 1]; pass 0 has no twiddles
+  template <int P>
+  __device__ __forceinline__ void fill(int j) {
+    if constexpr (P < NP) {
+      constexpr int R = pass_radix(LOGM, P), NS = pass_span(LOGM, P);
+#pragma unroll
+      for (int u = 0; u < nu<R, NS>(); ++u) {
+        const int k = (j + u * (M / 8)) % NS;
+        const c2 t1 = cis(-(float)k / (float)(NS * R));
+        c2 t = t1;
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+          w[P][u][r - 1] = t;
+          if (r + 1 < R) t = cmul(t, t1);
+        }
+      }
+      fill<P + 1>(j);
+    }
+  }
+  __device__ __forceinline__ explicit HwRegTwiddle(int j) { fill<1>(j); }
+  template <int MM, int R, int NS>
+  __device__ __forceinline__ c2 pass_tw(int u, int r, int) const {
+    static_assert(MM == M, "twiddles of another transform size");
+    return w[ilog2c(NS) / 3][nu<R, NS>() == 1 ? 0 : u][r - 1];
+  }
+};
+
 // Pass positions.  Input element u*R + r of a thread is index bj + r*M/R
 // (bj = j + u*M/8): the thread part j plus a constant; output element
 // u*R + r goes to (bj/NS)*NS*R + bj%NS + r*NS: a per-butterfly part plus the

@@ -19,9 +19,10 @@
 // FFT (fft_lds.h) plus the even/odd split; after the gains, the Hermitian
 // pre-processing and an N/2-point inverse FFT give two real output samples
 // per complex value.  W windows (one per M/8-thread slot) are transformed at
-// once, then their outputs are gathered into the tile accumulator position
-// by position in window order (atomic-free, deterministic).  The tile then
-// yields y, dL/dy = 2 (y - x)/T and its share of the loss sum (y - x)^2 / T.
+// once, and each slot adds its outputs from registers to the tile accumulator
+// (read, add, write; windows added at the same time do not overlap, so the
+// sum is atomic-free and its order fixed).  The tile then yields y,
+// dL/dy = 2 (y - x)/T and its share of the loss sum (y - x)^2 / T.
 //
 // k_stft_bwd: dL/dg_k = sum over windows (c_k/N) Re(X_k conj(E_k)), with X
 // the window's spectrum, E the spectrum of dL/dy over the window's outputs
@@ -33,8 +34,9 @@ namespace dgen {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kTile = 8192;   // output samples owned by a forward workgroup
-constexpr int kRounds = 8;    // window rounds per backward workgroup
+constexpr int kTile = 8192;   // output samples owned by a forward workgroup unless the op says fewer
+constexpr int kMinTile = 256;
+constexpr int kRounds = 8;    // window rounds per backward workgroup unless the op says fewer
 
 struct StftArgs {
   const float* x;      // [S][T]
@@ -45,45 +47,19 @@ struct StftArgs {
   float* dy;           // [S][T] or null
   float* lossp;        // [S][ntiles] or null
   float* gpart;        // [S][nblk][N/2 + 1] (backward)
-  int S, T, H, ntiles, nblk;
+  int S, T, H, ntiles, nblk, tile, rounds;
   float invT;
 };
 
 // Real N-point spectrum bins k and M-k (k = 0: bins 0 and M) from the
-// N/2-point complex transform Z of the even/odd-packed signal.
-__device__ __forceinline__ void split_bins(const SwzBuf& Z, int k, int M, float invN, c2& Xk, c2& Xm) {
-  const int km = (M - k) & (M - 1);
-  const c2 zk = Z[k], zm = Z[km];
+// N/2-point complex transform of the even/odd-packed signal: zk = Z[k],
+// zm = Z[(M-k) mod M], wk = exp(-2 pi i k / N).
+__device__ __forceinline__ void split_pair(c2 zk, c2 zm, int k, c2 wk, c2& Xk, c2& Xm) {
   const c2 e = {0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y)};
   const c2 o = {0.5f * (zk.y + zm.y), 0.5f * (zm.x - zk.x)};
-  const c2 wk = cis(-(float)k * invN);
   const c2 wo = cmul(wk, o);
   Xk = cadd(e, wo);
   Xm = k == 0 ? c2{e.x - o.x, 0.0f} : cconj(csub(e, wo));
-}
-
-// split_bins on values already read: zk = Z[k], zm = Z[(M-k) mod M].
-__device__ __forceinline__ void split_pair(c2 zk, c2 zm, int k, float invN, c2& Xk, c2& Xm) {
-  const c2 e = {0.5f * (zk.x + zm.x), 0.5f * (zk.y - zm.y)};
-  const c2 o = {0.5f * (zk.y + zm.y), 0.5f * (zm.x - zk.x)};
-  const c2 wk = cis(-(float)k * invN);
-  const c2 wo = cmul(wk, o);
-  Xk = cadd(e, wo);
-  Xm = k == 0 ? c2{e.x - o.x, 0.0f} : cconj(csub(e, wo));
-}
-
-// dst[0..n) = src[0..n): every load of the thread in flight before its LDS
-// writes (a loop that stored each load as it arrived waited out one memory
-// latency per iteration).
-template <int n>
-__device__ __forceinline__ void stage(float* dst, const float* __restrict__ src, int tid) {
-  constexpr int Q = (n + kThreads - 1) / kThreads;
-  float v[Q];
-#pragma unroll
-  for (int q = 0; q < Q; ++q) v[q] = src[min(tid + q * kThreads, n - 1)];
-#pragma unroll
-  for (int q = 0; q < Q; ++q)
-    if (tid + q * kThreads < n) dst[tid + q * kThreads] = v[q];
 }
 
 __device__ __forceinline__ float block_sum(float v, float* red) {
@@ -98,13 +74,22 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return t;
 }
 
-struct FwdLds {
-  float acc[kTile];
-  c2 buf[2048];
-  float gain[1025];
-  float red[kThreads / 64];
+// Two consecutive samples at a 4-byte aligned address, one 8-byte load.
+struct __attribute__((packed, aligned(4))) pair {
+  float x, y;
 };
 
+// What a round costs is its VALU instructions, so everything a thread uses
+// again every round (window values, pass and bin-pair twiddles) is in
+// registers (within three waves per SIMD), windows inside the signal load without bounds tests, and a slot
+// adds its outputs to the tile itself.  Slots take runs of consecutive
+// windows (slot q the q-th R of them, one a round), so that a round's windows
+// lie R hops apart: with R H >= N they do not overlap and one barrier a round
+// orders the adds.  Shorter tiles take consecutive windows a round and add
+// them in ceil(N/H) phases.  (Gathering a round's outputs position by
+// position, 16 x 4 masked LDS reads a thread whatever the hop, took half of a
+// round's 1200 instructions: 114 us at 8 x 2^20 samples, N = 1024, H = 256;
+// 83 us so.)
 template <int LOGN>
 __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
   constexpr int N = 1 << LOGN, M = N / 2, LOGM = LOGN - 1, P = M / 8, W = kThreads / P;
@@ -113,23 +98,31 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
   // bins need only wave-level ordering; the gather reads every slot
   constexpr bool WL = P <= 64;
   static_assert(W * M == 2048, "window slots must fill the FFT buffer");
-  __shared__ FwdLds L;
+  extern __shared__ __align__(16) float acc[];  // [tile]
+  __shared__ c2 lbuf[2048];
+  __shared__ float red[kThreads / 64];
+  __shared__ float gain[M + 1];
   const int tid = threadIdx.x, slot = tid / P, j = tid % P;
   const int s = blockIdx.y, tile = blockIdx.x, H = a.H;
-  const int a0 = tile * kTile, a1 = min(a.T, a0 + kTile);
+  const int a0 = tile * a.tile, a1 = min(a.T, a0 + a.tile);
   const float* xs = a.x + (size_t)s * a.T;
-  stage<M + 1>(L.gain, a.gains, tid);
-  for (int i = tid; i < kTile; i += kThreads) L.acc[i] = 0.0f;
+  for (int i = tid; i <= M; i += kThreads) gain[i] = a.gains[i];
+  for (int i = tid; i < a.tile; i += kThreads) acc[i] = 0.0f;
   // windows h = w*H with outputs [h, h+N) meeting [a0, a1)
   const int w_lo = a0 - N < 0 ? 0 : (a0 - N) / H + 1;
   const int w_hi = (a1 - 1) / H;
   const int nw = w_hi - w_lo + 1;
-  const SwzBuf buf(L.buf, slot * M);
+  const SwzBuf buf(lbuf, slot * M);
   const int sj = buf.part(j);
-  // after the inverse transform a slot's region holds its N real outputs in
-  // order: slot q's at zs + q * 2 * M
-  const float* zs = reinterpret_cast<const float*>(L.buf);
-  constexpr int kZStride = 2 * M;
+  const HwRegTwiddle<LOGM> tw(j);
+  // this thread's bin pairs k = j + u*P, M - k
+  c2 wp[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) wp[u] = cis(-(float)(j + u * P) / (float)N);
+  const int rounds = (nw + W - 1) / W, V = (N + H - 1) / H;
+  const bool runs = rounds >= V;  // a round's windows do not overlap
+  const int phases = runs ? 1 : min(V, W), phase = runs ? 0 : slot % V;
+  auto window = [&](int r) { return w_lo + (runs ? slot * rounds + r : r * W + slot); };
   constexpr float invN = 1.0f / (float)N;
   // the window values this thread multiplies (samples 2n, 2n+1 of its first
   // pass inputs n), in registers for every round
@@ -141,29 +134,62 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
   }
   // this thread's window samples of round r (element e of the first pass
   // needs samples 2n and 2n+1 of the window, n = in_pos(j, e)); the next
-  // round's are loaded while this one is transformed and gathered
+  // round's are loaded while this one is transformed
   float px[16];
-  auto fetch = [&](int r0) {
-    const int w = w_lo + r0 + slot;
-    const bool live = w <= w_hi;
-    const int h = w * H;
+  auto fetch = [&](int r) {
+    const int w = window(r), h = w * H, t00 = h - N + 1 + 2 * j;
+    if (__ballot(w > w_hi || h < N - 1) == 0) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const pair v = *reinterpret_cast<const pair*>(xs + t00 + 2 * in_off<M, pass_radix(LOGM, 0)>(e));
+        px[2 * e] = v.x;
+        px[2 * e + 1] = v.y;
+      }
+      return;
+    }
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const int n = in_pos<M, pass_radix(LOGM, 0)>(j, e);
-      const int t0 = h - N + 1 + 2 * n;
-      px[2 * e] = live && t0 >= 0 ? xs[t0] : 0.0f;
-      px[2 * e + 1] = live && t0 + 1 >= 0 ? xs[t0 + 1] : 0.0f;
+      const int t0 = t00 + 2 * in_off<M, pass_radix(LOGM, 0)>(e);
+      px[2 * e] = w <= w_hi && t0 >= 0 ? xs[t0] : 0.0f;
+      px[2 * e + 1] = w <= w_hi && t0 + 1 >= 0 ? xs[t0 + 1] : 0.0f;
+    }
+  };
+  // adds this thread's outputs of window w (complex output q holds samples
+  // 2q, 2q+1) to the tile
+  auto add = [&](int w, const c2 (&v)[8], const int (&op)[8]) {
+    const int h = w * H, o = h - a0;
+    const bool whole = w <= w_hi && o >= 0 && h + N <= a1;
+    if (__ballot(!whole) == 0 && H % 2 == 0) {
+#pragma unroll
+      for (int e0 = 0; e0 < 8; e0 += 4) {
+        float2 t[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[e] = *reinterpret_cast<const float2*>(acc + o + 2 * op[e0 + e]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          *reinterpret_cast<float2*>(acc + o + 2 * op[e0 + e]) =
+              float2{t[e].x + v[e0 + e].x * invN, t[e].y + v[e0 + e].y * invN};
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      return;
+    }
+    if (w > w_hi) return;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int i = o + 2 * op[e];
+      if (i >= 0 && i < a1 - a0) acc[i] += v[e].x * invN;
+      if (i + 1 >= 0 && i + 1 < a1 - a0) acc[i + 1] += v[e].y * invN;
     }
   };
   __syncthreads();
   fetch(0);
-  for (int r0 = 0; r0 < nw; r0 += W) {
+  for (int r = 0; r < rounds; ++r) {
     c2 v[8];
     int op[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = c2{px[2 * e] * hw[e].x, px[2 * e + 1] * hw[e].y};
-    fft<LOGM, false, WL>(buf, j, v, op);
-    if (r0 + W < nw) fetch(r0 + W);
+    fft<LOGM, false, WL>(buf, j, v, op, tw);
+    if (r + 1 < rounds) fetch(r + 1);
     fft_store<LOGM>(buf, j, v);
     lds_sync<WL>();
     // gains on the one-sided spectrum, then the Hermitian inverse
@@ -182,14 +208,14 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
       const int k = j + u * P;
       if (k > M / 2) continue;
       c2 Xk, Xm;
-      split_pair(zk[u], zm[u], k, invN, Xk, Xm);
-      const float gk = L.gain[k], gm = L.gain[M - k];
+      const c2 wk = wp[u];
+      split_pair(zk[u], zm[u], k, wk, Xk, Xm);
+      const float gk = gain[k], gm = gain[M - k];
       Xk = c2{Xk.x * gk, Xk.y * gk};
       Xm = c2{Xm.x * gm, Xm.y * gm};
       if (k == 0) {
         buf[0] = c2{Xk.x + Xm.x, Xk.x - Xm.x};
       } else {
-        const c2 wk = cis(-(float)k * invN);
         const c2 o1 = cmul(c2{Xk.x - Xm.x, Xk.y + Xm.y}, cconj(wk));
         buf[k] = c2{(Xk.x + Xm.x) - o1.y, (Xk.y - Xm.y) + o1.x};
         if (k != M - k) {
@@ -201,61 +227,11 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
     lds_sync<WL>();
     fft_load<LOGM>(buf, j, v);
     lds_sync<WL>();
-    fft<LOGM, true, WL>(buf, j, v, op);
-    // complex output q holds samples 2q, 2q+1 (unnormalised): scale by 1/N
-    float* zb = buf.raw();
-#pragma unroll
-    for (int e = 0; e < 8; ++e) *reinterpret_cast<float2*>(zb + 2 * op[e]) = float2{v[e].x * invN, v[e].y * invN};
-    lds_barrier();
-    // gather this round's windows into the tile, position by position
-    const int wb = w_lo + r0, hb = wb * H;
-    const int nq = min(W, w_hi - wb + 1);
-    const int span = (nq - 1) * H + N;
-    if constexpr (W <= 4) {
-      // span <= W*N = 4096 (H <= N): 16 positions per thread, gathered 4
-      // at a time with every slot read and accumulator read of a batch
-      // issued before its first sum (a position loop waited out LDS latency
-      // at every position); a slot that does not cover a position adds +0
-      // (exact)
-      constexpr int kPos = W * N / kThreads, kBatch = 4;
-#pragma unroll
-      for (int i0 = 0; i0 < kPos; i0 += kBatch) {
-        float z[kBatch][W], ac[kBatch];
-#pragma unroll
-        for (int b = 0; b < kBatch; ++b) {
-          const int p = tid + (i0 + b) * kThreads;
-#pragma unroll
-          for (int q = 0; q < W; ++q) {
-            const int ii = p - q * H;
-            const bool ok = q < nq && ii >= 0 && ii < N;
-            z[b][q] = zs[q * kZStride + (ok ? ii : 0)];
-            z[b][q] = ok ? z[b][q] : 0.0f;
-          }
-          ac[b] = L.acc[min(max(hb + p - a0, 0), kTile - 1)];
-        }
-#pragma unroll
-        for (int b = 0; b < kBatch; ++b) {
-          const int p = tid + (i0 + b) * kThreads, t = hb + p;
-          float sum = 0.0f;
-#pragma unroll
-          for (int q = 0; q < W; ++q) sum += z[b][q];
-          if (p < span && t >= a0 && t < a1) L.acc[t - a0] = ac[b] + sum;
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-      for (int p = tid; p < span; p += kThreads) {
-        const int t = hb + p;
-        if (t < a0 || t >= a1) continue;
-        float sum = 0.0f;
-        for (int q = 0; q < nq; ++q) {
-          const int i = p - q * H;
-          if (i >= 0 && i < N) sum += zs[q * kZStride + i];
-        }
-        L.acc[t - a0] += sum;
-      }
+    fft<LOGM, true, WL>(buf, j, v, op, tw);
+    for (int ph = 0; ph < phases; ++ph) {
+      if (phase == ph) add(window(r), v, op);
+      lds_barrier();
     }
-    lds_barrier();
   }
   float ls = 0.0f;
   // the tile's input samples are loaded 8 at a time, all in flight before use
@@ -267,7 +243,7 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
     for (int q = 0; q < 8; ++q) {
       const int t = t8 + q * kThreads;
       if (t >= a1) break;
-      const float yv = L.acc[t - a0];
+      const float yv = acc[t - a0];
       const float d = yv - xv[q];
       const size_t i = (size_t)s * a.T + t;
       if (a.y) a.y[i] = yv;
@@ -276,7 +252,7 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
     }
   }
   if (a.lossp) {
-    const float tot = block_sum(ls, L.red);
+    const float tot = block_sum(ls, red);
     if (tid == 0) a.lossp[(size_t)s * a.ntiles + tile] = tot * a.invT;
   }
 }
@@ -286,8 +262,10 @@ struct BwdLds {
   c2 aux[2048];
 };
 
+// (held to four waves per SIMD up to N = 1024: 53 -> 46 us at 8 x 2^20, N = 1024;
+// at 2048 that spills)
 template <int LOGN>
-__global__ __launch_bounds__(kThreads) void k_stft_bwd(StftArgs a) {
+__global__ __launch_bounds__(kThreads, LOGN <= 10 ? 4 : 2) void k_stft_bwd(StftArgs a) {
   constexpr int N = 1 << LOGN, M = N / 2, LOGM = LOGN - 1, P = M / 8, W = kThreads / P;
   constexpr int U = M / 2 / P + 1;  // bin pairs per thread
   constexpr bool WL = P <= 64;       // a window's threads lie in one wave
@@ -296,7 +274,7 @@ __global__ __launch_bounds__(kThreads) void k_stft_bwd(StftArgs a) {
   const int tid = threadIdx.x, slot = tid / P, j = tid % P;
   const int s = blockIdx.y, blk = blockIdx.x, H = a.H;
   const int nwin = (a.T + H - 1) / H;
-  const int wb = blk * kRounds * W, we = min(nwin, wb + kRounds * W);
+  const int wb = blk * a.rounds * W, we = min(nwin, wb + a.rounds * W);
   const float* xs = a.x + (size_t)s * a.T;
   const float* gs = a.dyin + (size_t)s * a.T;
   const SwzBuf buf(L.buf, slot * M);
@@ -309,6 +287,10 @@ __global__ __launch_bounds__(kThreads) void k_stft_bwd(StftArgs a) {
     hw[e] = float2{a.win[2 * n], a.win[2 * n + 1]};
   }
   constexpr float invN = 1.0f / (float)N;
+  const HwRegTwiddle<LOGM> tw(j);
+  c2 wp[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) wp[u] = cis(-(float)(j + u * P) / (float)N);
   float acc_k[U], acc_m[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) acc_k[u] = acc_m[u] = 0.0f;
@@ -322,17 +304,27 @@ __global__ __launch_bounds__(kThreads) void k_stft_bwd(StftArgs a) {
       // the window's outputs [h, h+N) (-> buf), transformed together
       c2 vx[8], vg[8];
       int op[8];
+      const int t00 = h - N + 1 + 2 * j, g00 = h + 2 * j;
+      if (__ballot(!live || h < N - 1 || h + N > a.T) == 0) {  // inside the signal: no bounds tests
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int n = in_pos<M, pass_radix(LOGM, 0)>(j, e);
-        const int t0 = h - N + 1 + 2 * n;
-        const float x0 = live && t0 >= 0 ? xs[t0] : 0.0f;
-        const float x1 = live && t0 + 1 >= 0 ? xs[t0 + 1] : 0.0f;
-        vx[e] = c2{x0 * hw[e].x, x1 * hw[e].y};
-        const int g0 = h + 2 * n;
-        vg[e] = c2{live && g0 < a.T ? gs[g0] : 0.0f, live && g0 + 1 < a.T ? gs[g0 + 1] : 0.0f};
+        for (int e = 0; e < 8; ++e) {
+          const int off = 2 * in_off<M, pass_radix(LOGM, 0)>(e);
+          const pair x = *reinterpret_cast<const pair*>(xs + t00 + off);
+          const pair g = *reinterpret_cast<const pair*>(gs + g00 + off);
+          vx[e] = c2{x.x * hw[e].x, x.y * hw[e].y};
+          vg[e] = c2{g.x, g.y};
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int off = 2 * in_off<M, pass_radix(LOGM, 0)>(e), t0 = t00 + off, g0 = g00 + off;
+          const float x0 = live && t0 >= 0 ? xs[t0] : 0.0f;
+          const float x1 = live && t0 + 1 >= 0 ? xs[t0 + 1] : 0.0f;
+          vx[e] = c2{x0 * hw[e].x, x1 * hw[e].y};
+          vg[e] = c2{live && g0 < a.T ? gs[g0] : 0.0f, live && g0 + 1 < a.T ? gs[g0 + 1] : 0.0f};
+        }
       }
-      fft2<LOGM, false, WL>(spec, buf, j, vx, vg, op);
+      fft2<LOGM, false, WL>(spec, buf, j, vx, vg, op, tw);
       fft_store<LOGM>(spec, j, vx);
       fft_store<LOGM>(buf, j, vg);
       lds_sync<WL>();
@@ -342,8 +334,9 @@ __global__ __launch_bounds__(kThreads) void k_stft_bwd(StftArgs a) {
       const int k = j + u * P;
       if (k > M / 2) break;
       c2 Xk, Xm, Ek, Em;
-      split_bins(spec, k, M, invN, Xk, Xm);
-      split_bins(buf, k, M, invN, Ek, Em);
+      const int km = (M - k) & (M - 1);
+      split_pair(spec[k], spec[km], k, wp[u], Xk, Xm);
+      split_pair(buf[k], buf[km], k, wp[u], Ek, Em);
       acc_k[u] += Xk.x * Ek.x + Xk.y * Ek.y;
       acc_m[u] += Xm.x * Em.x + Xm.y * Em.y;
     }
@@ -409,15 +402,15 @@ int stft_shape(int64_t S, int64_t T, int64_t N, int64_t H, int& logn, const char
 
 }  // namespace
 
-int stft_windows_per_block(int64_t N) { return kRounds * (kThreads * 16 / (int)N); }
-int stft_tile() { return kTile; }
-
 int launch_stft_fwd(const Launch& L, const dgen_hip_op& op) {
   const int64_t x = op.arg[0], win = op.arg[1], gains = op.arg[2], y = op.arg[3], dy = op.arg[4], lossp = op.arg[5];
   const int64_t S = op.arg[6], T = op.arg[7], N = op.arg[8], H = op.arg[9];
   int logn;
   if (int rc = stft_shape(S, T, N, H, logn, "stft_fwd")) return rc;
-  const int64_t ntiles = (T + kTile - 1) / kTile;
+  const int64_t tile = op.arg[10] ? op.arg[10] : kTile;
+  DGEN_REQUIRE(tile >= kMinTile && tile <= kTile, "stft_fwd: tile %lld outside [%d, %d]", (long long)tile, kMinTile,
+               kTile);
+  const int64_t ntiles = (T + tile - 1) / tile;
   DGEN_CHECK_CELL(L, x, S * T, "stft_fwd.x");
   DGEN_CHECK_CELL(L, win, N, "stft_fwd.window");
   DGEN_CHECK_CELL(L, gains, N / 2 + 1, "stft_fwd.gains");
@@ -437,8 +430,10 @@ int launch_stft_fwd(const Launch& L, const dgen_hip_op& op) {
   a.T = (int)T;
   a.H = (int)H;
   a.ntiles = (int)ntiles;
+  a.tile = (int)tile;
   a.invT = 1.0f / (float)T;
-  hipLaunchKernelGGL(fwd_kernel(logn), dim3((unsigned)ntiles, (unsigned)S), dim3(kThreads), 0, L.stream, a);
+  hipLaunchKernelGGL(fwd_kernel(logn), dim3((unsigned)ntiles, (unsigned)S), dim3(kThreads),
+                     (unsigned)(tile * sizeof(float)), L.stream, a);
   DGEN_LAUNCH_CHECK("k_stft_fwd");
   return 0;
 }
@@ -449,7 +444,9 @@ int launch_stft_bwd(const Launch& L, const dgen_hip_op& op) {
   int logn;
   if (int rc = stft_shape(S, T, N, H, logn, "stft_bwd")) return rc;
   const int64_t nwin = (T + H - 1) / H;
-  const int64_t wpb = stft_windows_per_block(N);
+  const int64_t rounds = op.arg[8] ? op.arg[8] : kRounds;
+  DGEN_REQUIRE(rounds >= 1 && rounds <= kRounds, "stft_bwd: rounds %lld outside [1, %d]", (long long)rounds, kRounds);
+  const int64_t wpb = rounds * (kThreads * 16 / N);
   const int64_t nblk = (nwin + wpb - 1) / wpb;
   DGEN_CHECK_CELL(L, x, S * T, "stft_bwd.x");
   DGEN_CHECK_CELL(L, win, N, "stft_bwd.window");
@@ -465,6 +462,7 @@ int launch_stft_bwd(const Launch& L, const dgen_hip_op& op) {
   a.T = (int)T;
   a.H = (int)H;
   a.nblk = (int)nblk;
+  a.rounds = (int)rounds;
   hipLaunchKernelGGL(bwd_kernel(logn), dim3((unsigned)nblk, (unsigned)S), dim3(kThreads), 0, L.stream, a);
   DGEN_LAUNCH_CHECK("k_stft_bwd");
   return 0;

@@ -28,7 +28,8 @@ MSS_TILE = 4096     # output samples per spectral-loss workgroup
 BQ_CHUNK = 512      # frames per biquad scan chunk (512 measured fastest of 128..1024)
 SVF_CHUNK = 256     # frames per SVF scan chunk
 SCAN_WAVES = 2048   # waves (64 lanes x one chunk) a filter scan's passes should have: two per SIMD
-STFT_TILE = 8192    # output samples per STFT forward workgroup
+STFT_TILE = 8192    # largest output tile of an STFT forward workgroup
+STFT_GROUPS = 512   # workgroups an STFT pass is split into if need be (two per CU)
 MEM_STEPS = 16      # membrane frames per time-blocked launch
 MEM_TILE = 32       # membrane cells per workgroup tile side
 MEM_WAVES = 16      # membrane waves per workgroup (4-row strips of a 64-row region)
@@ -837,9 +838,27 @@ class SweptPhasorSession:
 
 
 # ------------------------------------------------------------------ config 2
-def stft_windows_per_block(N: int) -> int:
-    """Windows summed by one gain-gradient workgroup (8 rounds of 4096/N)."""
-    return 8 * (4096 // N)
+def stft_tile(S: int, T: int, N: int, H: int) -> int:
+    """Output samples of a forward workgroup: STFT_TILE, halved (to no less
+    than 512) while that makes at most STFT_GROUPS workgroups.  A tile runs its
+    windows a few at a time, so a short signal wants short tiles on more of
+    the chip; a long one wants long tiles, whose edges repeat fewer windows.
+    (2 x 44101 samples, N = 512: 36 us at 8192, 7.5 at 512; 4 x 200000, N =
+    2048: 49 at 8192, 25 at 2048, 38 at 1024; 8 x 2^20, N = 1024: 86 at 8192, 96
+    at 4096.)"""
+    tile = STFT_TILE
+    while tile > 512 and S * ((T + tile // 2 - 1) // (tile // 2)) <= STFT_GROUPS:
+        tile //= 2
+    return tile
+
+
+def stft_rounds(S: int, nwin: int, N: int) -> int:
+    """Rounds of 4096 / N windows of a gain-gradient workgroup: 8, halved
+    while that makes at most STFT_GROUPS workgroups."""
+    rounds = 8
+    while rounds > 1 and S * ((nwin + rounds // 2 * (4096 // N) - 1) // (rounds // 2 * (4096 // N))) <= STFT_GROUPS:
+        rounds //= 2
+    return rounds
 
 
 def stft_program(cfg: StftConfig, train: bool = True, optimizer: bool = True) -> Program:
@@ -847,9 +866,12 @@ def stft_program(cfg: StftConfig, train: bool = True, optimizer: bool = True) ->
     sum (y - x)^2 / T against the raw input, gradient to the N/2+1 gains
     (``train``) and one Adam step (``optimizer``)."""
     S, T, N, H, nb = cfg.S, cfg.T, cfg.N, cfg.H, cfg.bins
-    ntiles = (T + STFT_TILE - 1) // STFT_TILE
+    tile = stft_tile(S, T, N, H)
+    ntiles = (T + tile - 1) // tile
     nwin = (T + H - 1) // H
-    nblk = (nwin + stft_windows_per_block(N) - 1) // stft_windows_per_block(N)
+    rounds = stft_rounds(S, nwin, N)
+    wpb = rounds * (4096 // N)
+    nblk = (nwin + wpb - 1) // wpb
     f4 = 4.0
     p = Program(max_frames=T)
     p.meta.update(cfg=cfg, ntiles=ntiles, nblk=nblk, train=train)
@@ -860,9 +882,9 @@ def stft_program(cfg: StftConfig, train: bool = True, optimizer: bool = True) ->
     lognn = float(np.log2(N))
     fft_flops = 2.5 * N * lognn  # one real N-point transform (split-radix estimate)
     windows = float(S * nwin)
-    halo = 1.0 + (N - H) / STFT_TILE  # windows recomputed at tile edges
+    halo = 1.0 + (N - H) / tile  # windows recomputed at tile edges
     if not train:
-        p.add(R.K_STFT_FWD, [x, win, g, y, -1, -1, S, T, N, H], label="stft_fwd",
+        p.add(R.K_STFT_FWD, [x, win, g, y, -1, -1, S, T, N, H, tile], label="stft_fwd",
               dispatch=f"tiles {ntiles}x{S}, windows {nwin}/signal", bytes=2.0 * S * T * f4,
               flops=windows * halo * 2 * fft_flops)
         p.output_cell = "y"
@@ -873,12 +895,12 @@ def stft_program(cfg: StftConfig, train: bool = True, optimizer: bool = True) ->
     gpart = p.alloc("grad_partials", S * nblk * nb)
     G = p.alloc("grads", nb)
     ws = p.alloc("colsum_ws", max(_colsum_ws(S * ntiles, 1), _colsum_ws(S * nblk, nb)))
-    p.add(R.K_STFT_FWD, [x, win, g, y, dy, lossp, S, T, N, H], label="stft_fwd",
+    p.add(R.K_STFT_FWD, [x, win, g, y, dy, lossp, S, T, N, H, tile], label="stft_fwd",
           dispatch=f"tiles {ntiles}x{S}, windows {nwin}/signal", bytes=3.0 * S * T * f4,
           flops=windows * halo * 2 * fft_flops)
     p.add(R.K_COLSUM, [lossp, loss, S * ntiles, 1, 1, ws], label="loss_sum", dispatch="chunkPartialsReduceToCell",
           bytes=(S * ntiles + 1) * f4, flops=float(S * ntiles))
-    p.add(R.K_STFT_BWD, [x, win, dy, gpart, S, T, N, H], label="stft_bwd",
+    p.add(R.K_STFT_BWD, [x, win, dy, gpart, S, T, N, H, rounds], label="stft_bwd",
           dispatch=f"window runs {nblk}x{S}", bytes=2.0 * S * T * f4 + S * nblk * nb * f4,
           flops=windows * (2 * fft_flops + 4 * nb))
     p.add(R.K_COLSUM, [gpart, G, S * nblk, nb, nb, ws], label="grad_sum", dispatch="chunkPartialsReduceToCell",

@@ -9,6 +9,8 @@ import pytest
 
 import oracle as O
 from dgen_hip import StftConfig
+from dgen_hip import runtime as R
+from dgen_hip.program import Program
 from dgen_hip.programs import StftSession, stft_program
 from dgen_hip.runtime import HIPLazyRuntime
 
@@ -143,3 +145,38 @@ def test_full_configuration_matches_oracle(gpu):
     e = np.linalg.norm(g - g64) / np.linalg.norm(g64)
     print(f"grad rel L2 err {e:.2e}, max abs {np.abs(g - g64).max():.2e} of max {np.abs(g64).max():.2e}")
     assert e < 1e-4
+
+
+@pytest.mark.parametrize("S,T,N,H", [(2, 9001, 64, 16), (1, 5000, 64, 1), (2, 9001, 128, 33), (3, 20000, 256, 64),
+                                     (1, 20003, 512, 171), (2, 30001, 1024, 256), (1, 9000, 1024, 100),
+                                     (2, 20000, 2048, 512), (1, 9000, 2048, 2048)])
+@pytest.mark.parametrize("tile,rounds", [(256, 1), (512, 2), (1280, 3), (8192, 8)])
+def test_tiles_and_rounds_agree_with_the_oracle(gpu, S, T, N, H, tile, rounds):
+    """Output tiles and gradient runs of any length: windows added in phases
+    (tiles shorter than the windows of a round span) or a run per slot, odd
+    hops and tiles, hops of 1 and of N.  A position's sum of up to N/H windows
+    is only reordered, so y keeps test_forward_matches_oracle's bar and the
+    loss and gradient the fp32 oracle's distance from fp64."""
+    cfg = StftConfig(S=S, T=T, N=N, H=H)
+    x, g = cfg.inputs(), random_gains(cfg.bins, N + T)
+    print(f"case S={S} T={T} N={N} H={H} tile={tile} rounds={rounds}", flush=True)
+    p = Program(max_frames=T)
+    nb, nt = cfg.bins, -(-T // tile)
+    nblk = -(-(-(-T // H)) // (rounds * (4096 // N)))
+    c = {n: p.alloc(n, k) for n, k in (("x", S * T), ("window", N), ("gains", nb), ("y", S * T), ("dy", S * T),
+                                       ("lossp", S * nt), ("gpart", S * nblk * nb))}
+    p.add(R.K_STFT_FWD, [c["x"], c["window"], c["gains"], c["y"], c["dy"], c["lossp"], S, T, N, H, tile])
+    p.add(R.K_STFT_BWD, [c["x"], c["window"], c["dy"], c["gpart"], S, T, N, H, rounds])
+    with HIPLazyRuntime(p) as rt:
+        for n, a in (("x", x), ("window", cfg.window()), ("gains", g)):
+            rt.write(n, a)
+        for _ in range(2):
+            rt.runNoCopy()
+        y, loss = rt.read("y").reshape(S, T), rt.read("lossp").astype(np.float64).sum()
+        dg = rt.read("gpart").reshape(-1, nb).astype(np.float64).sum(0)
+    l32, g32, y32 = O.stft_step(x, N, H, cfg.window(), g, want_y=True, prec="f32")
+    l64, g64, y64 = O.stft_step(x, N, H, cfg.window(), g, want_y=True, prec="f64")
+    assert np.abs(y - y64).max() <= 8.0 * np.abs(y32 - y64).max() + 2e-6
+    assert abs(loss - l64) <= 8.0 * abs(l32 - l64) + 2e-6 * abs(l64)
+    n = np.linalg.norm
+    assert n(dg - g64) <= 8.0 * n(g32 - g64) + 2e-6 * n(g64)
