@@ -164,6 +164,62 @@ static int colsum_chunks(int64_t rows, int nw = 0) {
 }
 
 // out_q (q < nw) rows of out0 (stride ld_out0) and the plain sum into plain_out.
+// Few rows: the two stages in one launch, a workgroup of 16 waves per 64
+// columns.  What stage 1's wave w of row chunk c sums is summed here by wave
+// (4c + w) % 16, and the sums are added in the stages' order, so the result is
+// theirs bit for bit.  The second launch costs more than it saves there:
+// 5.2-5.8 us for 256 x 24 to 512 x 1024, 2.6-3.8 us in one.
+constexpr int kColOneRows = 512;
+constexpr int kColOneChunks = kColOneRows / 32;
+constexpr int64_t kColOneCells = 1 << 19;  // more is worth the second launch's wider grid
+__global__ __launch_bounds__(1024) void k_colsum_one(const float* __restrict__ A, int lda, int rows, int cols,
+                                                     int chunks, int chunk, float* __restrict__ out) {
+  __shared__ float red[4 * kColOneChunks][64];
+  __shared__ float fin[4][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int n = blockIdx.x * 64 + lane;
+  const float* col = A + min(n, cols - 1);
+  constexpr int kR = 8;  // rows loaded at once
+  for (int pr = wave; pr < 4 * chunks; pr += 16) {
+    const int m0 = (pr >> 2) * chunk, m1 = min(rows, m0 + chunk);
+    float acc = 0.f;
+    for (int m = m0 + (pr & 3); m < m1; m += 4 * kR) {
+      float v[kR];
+#pragma unroll
+      for (int i = 0; i < kR; ++i) v[i] = col[(size_t)min(m + 4 * i, m1 - 1) * lda];
+#pragma unroll
+      for (int i = 0; i < kR; ++i) acc = m + 4 * i < m1 ? acc + v[i] : acc;
+    }
+    red[pr][lane] = acc;
+  }
+  __syncthreads();
+  if (wave < 4) {
+    float s = 0.f;
+    for (int c = wave; c < chunks; c += 4)
+      s += ((red[4 * c][lane] + red[4 * c + 1][lane]) + red[4 * c + 2][lane]) + red[4 * c + 3][lane];
+    fin[wave][lane] = s;
+  }
+  __syncthreads();
+  if (wave == 0 && n < cols) out[n] = ((fin[0][lane] + fin[1][lane]) + fin[2][lane]) + fin[3][lane];
+}
+
+// One column of consecutive values: one workgroup, 1024 values at a time.
+constexpr int kSumOneRows = 16384;
+__global__ __launch_bounds__(1024) void k_sum_one(const float* __restrict__ A, int rows, float* __restrict__ out) {
+  __shared__ float red[16];
+  float acc = 0.f;
+#pragma unroll 8
+  for (int m = threadIdx.x; m < rows; m += 1024) acc += A[m];
+  acc = wave_sum(acc);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    float t = 0.f;
+    for (int w = 0; w < 16; ++w) t += red[w];
+    out[0] = t;
+  }
+}
+
 static int colsum_launch(const Launch& L, const float* A, int lda, const float* X, int nw, int rows, int cols,
                          float* ws, float* out0, int ld_out0, float* plain_out) {
   const int chunks = colsum_chunks(rows, nw);
@@ -193,6 +249,17 @@ int launch_colsum(const Launch& L, const dgen_hip_op& op) {
   DGEN_CHECK_CELL(L, out, cols, "colsum.out");
   DGEN_CHECK_CELL(L, ws, (int64_t)chunks * cols, "colsum.workspace");
   if (L.dry) return 0;
+  if (cols == 1 && lda == 1 && rows <= kSumOneRows) {
+    hipLaunchKernelGGL(k_sum_one, dim3(1), dim3(1024), 0, L.stream, cell(L, A), (int)rows, cell(L, out));
+    DGEN_LAUNCH_CHECK("k_sum_one");
+    return 0;
+  }
+  if (rows <= kColOneRows && rows * cols <= kColOneCells) {
+    hipLaunchKernelGGL(k_colsum_one, dim3((unsigned)((cols + 63) / 64)), dim3(1024), 0, L.stream, cell(L, A), (int)lda,
+                       (int)rows, (int)cols, chunks, (int)((rows + chunks - 1) / chunks), cell(L, out));
+    DGEN_LAUNCH_CHECK("k_colsum_one");
+    return 0;
+  }
   return colsum_launch(L, cell(L, A), (int)lda, nullptr, 0, (int)rows, (int)cols, cell(L, ws), nullptr, 0,
                        cell(L, out));
 }
@@ -373,11 +440,13 @@ int launch_heads_bwd(const Launch& L, const dgen_hip_op& op) {
 // Adam.step (Optimizers.swift:164-204): t += 1; bias corrections in fp32;
 // m = b1 m + (1-b1) g; v = b2 v + (1-b2) g g; p -= lr mhat / (sqrt(vhat)+eps).
 // The step counter lives in a device cell; it is read by every thread and
-// incremented afterwards by a separate one-thread launch (stream order).
+// incremented afterwards: by a separate one-thread launch (stream order), or,
+// where one workgroup holds all parameters (ONE), by that workgroup.
+constexpr int64_t kAdamOne = 4096;  // parameters of the one-workgroup form
 #pragma clang fp contract(off)
+template <bool ONE>
 __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, size_t n, const float* __restrict__ tcell, float lr, float b1, float b2,
-                       float eps) {
+                       float* __restrict__ v, size_t n, float* tcell, float lr, float b1, float b2, float eps) {
   const float t = tcell[0] + 1.0f;
   const float bc1 = 1.0f - powf(b1, t);
   const float bc2 = 1.0f - powf(b2, t);
@@ -389,6 +458,10 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
     p[j] = p[j] - lr * mh / (sqrtf(vh) + eps);
     m[j] = mj;
     v[j] = vj;
+  }
+  if constexpr (ONE) {
+    __syncthreads();  // every thread has read the counter
+    if (threadIdx.x == 0) tcell[0] = t;
   }
 }
 #pragma clang fp contract(on)
@@ -406,8 +479,14 @@ int launch_adam(const Launch& L, const dgen_hip_op& op) {
   DGEN_CHECK_CELL(L, V, n, "adam.v");
   DGEN_CHECK_CELL(L, tc, 1, "adam.step");
   if (L.dry) return 0;
+  if (n <= kAdamOne) {
+    hipLaunchKernelGGL(k_adam<true>, dim3(1), dim3(1024), 0, L.stream, cell(L, P), cell(L, G), cell(L, M), cell(L, V),
+                       (size_t)n, cell(L, tc), op.farg[0], op.farg[1], op.farg[2], op.farg[3]);
+    DGEN_LAUNCH_CHECK("k_adam");
+    return 0;
+  }
   unsigned blocks = (unsigned)std::min<int64_t>((n + 255) / 256, (int64_t)L.cu_count * 8);
-  hipLaunchKernelGGL(k_adam, dim3(blocks), dim3(256), 0, L.stream, cell(L, P), cell(L, G), cell(L, M), cell(L, V),
+  hipLaunchKernelGGL(k_adam<false>, dim3(blocks), dim3(256), 0, L.stream, cell(L, P), cell(L, G), cell(L, M), cell(L, V),
                      (size_t)n, cell(L, tc), op.farg[0], op.farg[1], op.farg[2], op.farg[3]);
   DGEN_LAUNCH_CHECK("k_adam");
   hipLaunchKernelGGL(k_increment, dim3(1), dim3(64), 0, L.stream, cell(L, tc));
