@@ -737,6 +737,226 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
                       C, ldc, epi, bias, aux, ldaux, nullptr, cs, cw, ncw);
 }
 
+// Split-bf16 GEMM for few tiles: the products, k-steps, accumulation order and
+// epilogues of k_gemm_x6, so its results bit for bit, on 128 x 32 tiles of two
+// waves that read their fragments from global memory straight into registers,
+// kSmDepth k-steps ahead, with no LDS and no barrier in the k-loop.  With few
+// 128 x 128 tiles the chip is empty and a tile lasts as long as its k-steps'
+// load latencies one after the other, 1.5 us each; here 0.7.  The price is
+// that nothing is shared: every wave splits its own operands (132 VALU
+// instructions a k-step beside 12 MFMAs).  us, before and now, by 128 x 128
+// tiles (times k-splits): forward K = 512, 12 tiles 48.4 / 26.9, 64 47.7 / 30.6,
+// 128 45.5 / 38.6, 252 52.1 / 57.2; weight gradients, 2 92.1 / 38.7, 16 89.8 /
+// 38.9, 64 70.9 / 43.2, 128 74.1 / 67.0, 256 82.0 / 89.2: up to kSmTiles.
+constexpr int kSmDepth = 4;
+constexpr int64_t kSmTiles = 128;
+template <bool A_KMAJ, bool B_NK, bool BPL, bool VEC>
+__global__ __launch_bounds__(128) void k_gemm_x6s(const float* __restrict__ A, const float* __restrict__ B,
+                                                  float* __restrict__ C, int M, int N, int K, int lda, int ldb,
+                                                  int ldc, int epi, const float* __restrict__ bias,
+                                                  const float* __restrict__ aux, int ldaux, int kchunk,
+                                                  float* __restrict__ ws, float* __restrict__ cs,
+                                                  const float* __restrict__ cw, int ncw,
+                                                  const uint4* __restrict__ bpl, int K8) {
+  constexpr int BK = 16;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = lane >> 5, r = lane & 31;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * 32, wm = wave * 64;
+  const int kbeg = blockIdx.z * kchunk, kend = min(K, kbeg + kchunk);
+  const int col = n0 + r, colc = min(col, N - 1);
+  int rows[2];  // clamped: what lies past M is not stored
+#pragma unroll
+  for (int t = 0; t < 2; ++t) rows[t] = min(m0 + wm + 32 * t + r, M - 1);
+
+  // k-values k0 + 8h .. + 7 of one row (or column) of an operand.  off: the
+  // lane's byte offset of its first value at k-step 0, to which a whole
+  // k-step's loads add a uniform address.
+  auto off_of = [&](bool kmaj, int line, int ld) {
+    return 4u * (unsigned)(kmaj ? 8 * h * ld + line : line * ld + 8 * h);
+  };
+  auto at = [](const float* base, unsigned off) {
+    return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + off);
+  };
+  auto load8 = [&](const float* X, bool kmaj, unsigned off, int ld, int k0, float (&x)[8]) {
+    if (kmaj) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = *at(X + (size_t)(k0 + j) * ld, off);
+    } else if (VEC) {
+      const float* q = at(X + k0, off);
+      const float4 u = *reinterpret_cast<const float4*>(q), w = *reinterpret_cast<const float4*>(q + 4);
+      x[0] = u.x; x[1] = u.y; x[2] = u.z; x[3] = u.w;
+      x[4] = w.x; x[5] = w.y; x[6] = w.z; x[7] = w.w;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = *at(X + k0 + j, off);
+    }
+  };
+  // the last, partial k-step: clamped, zero past kend
+  auto tail8 = [&](const float* X, bool kmaj, int line, int ld, int k0, float (&x)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int kk = k0 + 8 * h + j, k = min(kk, kend - 1);
+      const float v = kmaj ? X[(size_t)k * ld + line] : X[(size_t)line * ld + k];
+      x[j] = kk < kend ? v : 0.f;
+    }
+  };
+  const unsigned aoff[2] = {off_of(A_KMAJ, rows[0], lda), off_of(A_KMAJ, rows[1], lda)};
+  const unsigned boff = BPL ? 0u : off_of(!B_NK, colc, ldb);
+  struct Step {
+    float a[2][8], b[BPL ? 1 : 8];
+    uint4 p[BPL ? 3 : 1];
+  };
+  auto load_planes = [&](int k0, Step& s) {
+    const int kg = (k0 >> 3) + h;
+    const size_t plane = (size_t)K8 * N;
+    const unsigned po = (unsigned)(min(kg, K8 - 1) * N + colc);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const uint4 v = (bpl + q * plane)[po];
+      s.p[q] = kg < K8 ? v : make_uint4(0u, 0u, 0u, 0u);
+    }
+  };
+  auto load = [&](int k0, Step& s) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) load8(A, A_KMAJ, aoff[t], lda, k0, s.a[t]);
+    if constexpr (BPL) load_planes(k0, s);
+    else load8(B, !B_NK, boff, ldb, k0, s.b);
+  };
+  floatx16 acc[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
+  auto step = [&](const Step& s) {
+    bf16x8 fa[2][3], fb[3];
+    uint4 p0, p1, p2;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      split8(s.a[t], p0, p1, p2);
+      fa[t][0] = __builtin_bit_cast(bf16x8, p0);
+      fa[t][1] = __builtin_bit_cast(bf16x8, p1);
+      fa[t][2] = __builtin_bit_cast(bf16x8, p2);
+    }
+    if constexpr (BPL) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) fb[q] = __builtin_bit_cast(bf16x8, s.p[q]);
+    } else {
+      split8(s.b, p0, p1, p2);
+      fb[0] = __builtin_bit_cast(bf16x8, p0);
+      fb[1] = __builtin_bit_cast(bf16x8, p1);
+      fb[2] = __builtin_bit_cast(bf16x8, p2);
+    }
+    constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[t][pa[q]], fb[pb[q]], acc[t], 0, 0, 0);
+  };
+  // whole k-steps, kSmDepth ahead (past the last one it is loaded again)
+  const int nf = max(0, kend - kbeg) / BK;
+  if (nf > 0) {
+    Step buf[kSmDepth];
+    auto fetch = [&](int i, Step& s) { load(kbeg + min(i, nf - 1) * BK, s); };
+#pragma unroll
+    for (int d = 0; d < kSmDepth; ++d) fetch(d, buf[d]);
+    int i = 0;
+    for (; i + kSmDepth <= nf; i += kSmDepth)
+#pragma unroll
+      for (int d = 0; d < kSmDepth; ++d) {
+        step(buf[d]);
+        fetch(i + d + kSmDepth, buf[d]);
+      }
+#pragma unroll
+    for (int d = 0; d < kSmDepth - 1; ++d)
+      if (i + d < nf) step(buf[d]);
+  }
+  if (kbeg + nf * BK < kend) {
+    Step t;
+    const int k0 = kbeg + nf * BK;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) tail8(A, A_KMAJ, rows[q], lda, k0, t.a[q]);
+    if constexpr (BPL) load_planes(k0, t);
+    else tail8(B, !B_NK, colc, ldb, k0, t.b);
+    step(t);
+  }
+
+  // gemm_epilogue on this tile (accumulator layout as there)
+  auto row_of = [&](int t, int v) { return m0 + wm + t * 32 + (v >> 2) * 8 + h * 4 + (v & 3); };
+  if (!ws && epi == EPI_TANH_GRAD) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      float hv[16];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int row = row_of(t, v);
+        hv[v] = (row < M && col < N) ? aux[(size_t)row * ldaux + col] : 0.f;
+      }
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int row = row_of(t, v);
+        acc[t][v] *= 1.f - hv[v] * hv[v];
+        // rows past M were loaded as copies of the last one: zero them, as
+        // the column sums below expect
+        if (row >= M) acc[t][v] = 0.f;
+        if (row < M && col < N) C[(size_t)row * ldc + col] = acc[t][v];
+      }
+    }
+    if (cs) {
+      __shared__ float red[5][2][32];
+      __shared__ __align__(16) float wt[4][BM];
+      if (ncw) {
+        for (int i = threadIdx.x; i < ncw * BM; i += 128) {
+          const int rr = i / ncw, q = i - rr * ncw;
+          wt[q][rr] = m0 + rr < M ? cw[(size_t)m0 * ncw + i] : 0.f;
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int q = 0; q < ncw; ++q) {
+          const float* wq = &wt[q][wm + h * 4];
+          float s = 0.f;
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+              const float4 w = *reinterpret_cast<const float4*>(wq + t * 32 + g * 8);
+              s = fmaf(w.x, acc[t][g * 4 + 0], s);
+              s = fmaf(w.y, acc[t][g * 4 + 1], s);
+              s = fmaf(w.z, acc[t][g * 4 + 2], s);
+              s = fmaf(w.w, acc[t][g * 4 + 3], s);
+            }
+          s += __shfl_xor(s, 32, 64);
+          if (lane < 32) red[q][wave][lane] = s;
+        }
+      }
+      float s = 0.f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) s += row_of(t, v) < M ? acc[t][v] : 0.f;
+      s += __shfl_xor(s, 32, 64);
+      if (lane < 32) red[ncw][wave][lane] = s;
+      __syncthreads();
+      if (wave == 0 && lane < 32 && col < N)
+        for (int q = 0; q <= ncw; ++q)
+          cs[((size_t)blockIdx.y * (ncw + 1) + q) * N + col] = red[q][0][lane] + red[q][1][lane];
+    }
+    return;
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int row = row_of(t, v);
+      if (row >= M || col >= N) continue;
+      const float a = acc[t][v];
+      if (ws) ws[((size_t)blockIdx.z * M + row) * N + col] = a;
+      else if (epi == EPI_BIAS_TANH) C[(size_t)row * ldc + col] = fast_tanh(a + bias[col]);
+      else if (epi == EPI_BIAS) C[(size_t)row * ldc + col] = a + bias[col];
+      else C[(size_t)row * ldc + col] = a;
+    }
+}
+
 // Three bfloat16 planes of an fp32 matrix, for an operand that many tiles
 // of the split-bf16 GEMM share (the weights): value (k, n) at
 // src[k*ldk + n*ldn] (0 <= k < K, 0 <= n < N) goes to plane p at
@@ -963,7 +1183,22 @@ int launch_gemm(const Launch& L, const dgen_hip_op& op) {
 #define DGEN_X6L(AK_, BT_)                                                                                          \
   launch_x6<AK_, BT_>(va, vb, full6, g, L.stream, pa, pb, pc, M, N, K, lda, ldb, ldc, e, pbias, paux, ldaux, kchunk, \
                       pws, pcs, pcw, ncw, pbpl, (int)K8)
-    if (pbpl && full6 && alay == 0 && splits == 1 && K % 32 == 0 && (int64_t)M * lda < (1ll << 32) &&
+    if ((int64_t)g.x * g.y * g.z <= kSmTiles && ext_a < (1ll << 31) && (pbpl || ext_b < (1ll << 31))) {
+      const dim3 gs((unsigned)((N + 31) / 32), g.y, g.z);
+      auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, gs, dim3(128), 0, L.stream, pa, pb, pc, (int)M, (int)N, (int)K, (int)lda, (int)ldb,
+                           (int)ldc, e, pbias, paux, (int)ldaux, (int)kchunk, pws, pcs, pcw, ncw, pbpl, (int)K8);
+      };
+      // operands stored along k load four values at a time when aligned
+      const bool v = (alay || va) && (pbpl || !blay || vb);
+      if (pbpl) {
+        if (alay) go(k_gemm_x6s<true, false, true, true>);
+        else v ? go(k_gemm_x6s<false, false, true, true>) : go(k_gemm_x6s<false, false, true, false>);
+      } else if (alay && !blay) go(k_gemm_x6s<true, false, false, true>);
+      else if (alay) v ? go(k_gemm_x6s<true, true, false, true>) : go(k_gemm_x6s<true, true, false, false>);
+      else if (blay) v ? go(k_gemm_x6s<false, true, false, true>) : go(k_gemm_x6s<false, true, false, false>);
+      else v ? go(k_gemm_x6s<false, false, false, true>) : go(k_gemm_x6s<false, false, false, false>);
+    } else if (pbpl && full6 && alay == 0 && splits == 1 && K % 32 == 0 && (int64_t)M * lda < (1ll << 32) &&
         3 * K8 * N < (1ll << 32)) {
       hipLaunchKernelGGL(k_gemm_x6d, g, dim3(256), 0, L.stream, pa, pc, (int)M, (int)N, (int)K, (int)lda, (int)ldc, e,
                          pbias, paux, (int)ldaux, pcs, pcw, ncw, pbpl, (int)K8);

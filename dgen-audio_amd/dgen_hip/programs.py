@@ -23,6 +23,7 @@ MAX_HARMONICS = 256  # the synth kernels' harmonic groups (four of 64)
 MAX_CONTROLS = 512   # control columns K + 2 + NF
 SPLITK_ROWS = 1024  # rows per split of the weight-gradient GEMMs
 GEMM_TILE_M = 128  # output rows per GEMM workgroup tile (k_gemm.hip BM)
+GEMM_SMALL_TILES = 128  # 128 x 128 tiles up to which a split-bf16 GEMM splits its own operands (k_gemm.hip kSmTiles)
 SPLITK_ROWS_HEADS = 256  # the heads' weight gradient has one 128-wide column tile: split finer to fill the chip
 MSS_TILE = 4096     # output samples per spectral-loss workgroup
 BQ_CHUNK = 512      # frames per biquad scan chunk (512 measured fastest of 128..1024)
@@ -204,11 +205,17 @@ def harmonic_program(cfg: HarmonicConfig, train: bool = True, optimizer: bool = 
     # the heads' data gradient runs over NC rounded up to 32 (dZ's padding
     # columns are zero, and so are the planes' rows past NC), so its tiles
     # take the pipelined full-tile kernel (whole k-steps of 32)
-    kh = NC if gm == 0 else min(LDC, (NC + 31) // 32 * 32)
-    if gm == 1:
+    # GEMMs of few tiles split their operands themselves (GEMM_SMALL_TILES) and
+    # take no planes: a launch per operand would cost more
+    mt = (M + GEMM_TILE_M - 1) // GEMM_TILE_M
+    few = lambda n: mt * ((n + GEMM_TILE_M - 1) // GEMM_TILE_M) <= GEMM_SMALL_TILES  # noqa: E731
+    pl_hid, pl_fwdh = gm == 1 and not few(Hd), gm == 1 and not few(NC)
+    kh = min(LDC, (NC + 31) // 32 * 32) if pl_hid else NC
+    if pl_hid:
         for l in range(1, Lyr):
             W, _b = woff[l]
             fwd_pl[l] = _split_planes(p, f"W{l + 1}_planes", W, Hd, Hd, Hd, 1)
+    if pl_fwdh:
         fwd_plh = _split_planes(p, "Wh_planes", Wh, Hd, NC, NC, 1)
     for l in range(1, Lyr):
         W, b = woff[l]
@@ -221,7 +228,7 @@ def harmonic_program(cfg: HarmonicConfig, train: bool = True, optimizer: bool = 
           dispatch="gemm", bytes=(M * Hd + Hd * NC + NC + M * NC) * f4, flops=2.0 * M * Hd * NC, bound=mfma)
     p.add(R.K_HEADS_FWD, [Z, ctrl, M, K, NF, LDC], label="heads", dispatch=f"perFrameScaled({M})",
           bytes=2 * M * NC * f4, flops=M * (K * 12.0 + NF * 8.0))
-    if gm == 1 and train:
+    if pl_hid and train:
         # the data gradients' W^T planes: after the control network, where
         # stream 0 waits for the phase chain, not before the forward GEMMs
         for l in range(1, Lyr):
@@ -335,7 +342,6 @@ def harmonic_program(cfg: HarmonicConfig, train: bool = True, optimizer: bool = 
     # the first layer the tile also writes the sums weighted by each input
     # column of X, so W1 and b1 (contiguous in the parameters) reduce
     # together from (din + 1) partial rows per tile.
-    mt = (M + GEMM_TILE_M - 1) // GEMM_TILE_M
     if din > 4:
         raise ValueError(f"first-layer fan-in {din} > 4")
     dcol = [p.alloc(f"dZ{l + 1}_tile_colsums", mt * (din + 1 if l == 0 else 1) * Hd) for l in range(Lyr)]

@@ -191,3 +191,57 @@ def test_product_mode_is_validated(gpu):
     with pytest.raises(Exception):
         with R.HIPLazyRuntime(p, 0) as rt:
             rt.runNoCopy()
+
+
+FEW = {  # M, N, K, A layout, B layout, epilogue, split, planes, column partials' weights (-1: none)
+    "forward": (375, 96, 96, 0, 0, 2, 1, True, -1),
+    "forward, unaligned k": (130, 59, 97, 0, 0, 1, 1, False, -1),
+    "one value": (1, 1, 1, 0, 0, 0, 1, False, -1),
+    "k of one step less one": (33, 31, 15, 0, 1, 1, 1, False, -1),
+    "four steps and a tail": (64, 128, 67, 1, 1, 0, 1, False, -1),
+    "weight gradient": (96, 59, 375, 1, 0, 0, 1, False, -1),
+    "split": (256, 100, 1000, 1, 0, 0, 4, False, -1),
+    "data gradient": (256, 96, 59, 0, 1, 3, 1, True, 0),
+    "data gradient, weighted sums": (384, 130, 64, 0, 1, 3, 1, False, 4),
+}
+
+
+@pytest.mark.parametrize("name", list(FEW))
+def test_few_tiles_give_the_large_kernel_bit_for_bit(gpu, name):
+    """Launches of few tiles keep the k-steps and the order of the partial
+    products, so a product equals the same rows of one tall enough for the
+    128 x 128 kernel, column partials of whole tiles included."""
+    M, N, K, al, bl, epi, split, planes, nw = FEW[name]
+    tall = 128 * (130 // ((N + 127) // 128 * split) + 1)
+    rng = np.random.default_rng(M + N + K)
+    a = rng.standard_normal((tall, K)).astype(np.float32)
+    b = rng.standard_normal((K, N)).astype(np.float32)
+    bias, cw = rng.standard_normal(N).astype(np.float32), rng.standard_normal((tall, 4)).astype(np.float32)
+    aux = np.tanh(rng.standard_normal((tall, N))).astype(np.float32)
+
+    def run(m):
+        p = Program(max_frames=1)
+        mt, K8, w = -(-m // 128), (K + 7) // 8, max(nw, 0)
+        c = {k: p.alloc(k, n) for k, n in (("a", m * K), ("b", K * N), ("c", m * N), ("bias", N), ("aux", m * N),
+                                           ("cw", max(1, m * w)), ("cs", mt * (w + 1) * N), ("ws", split * m * N),
+                                           ("pl", 3 * K8 * N * 4))}
+        lda, ldb = (m if al else K), (K if bl else N)
+        if planes:
+            p.add(R.K_SPLIT_BF16, [c["b"], c["pl"], K, N, 1 if bl else N, K if bl else 1])
+        p.add(R.K_GEMM, [c["a"], c["b"], c["c"], m, N, K, lda, ldb, N, al, bl, epi, c["bias"] if epi in (1, 2) else -1,
+                         c["aux"] if epi == 3 else -1, N, split, c["ws"], c["cs"] if nw >= 0 else -1,
+                         c["cw"] if w else -1, w, 1, c["pl"] if planes else -1])
+        with R.HIPLazyRuntime(p) as rt:
+            rt.write("a", a[:m].T if al else a[:m])
+            rt.write("b", b.T if bl else b)
+            rt.write("bias", bias)
+            rt.write("aux", aux[:m])
+            if w:
+                rt.write("cw", cw[:m, :w])
+            rt.runNoCopy()
+            return rt.read("c").reshape(m, N), rt.read("cs").reshape(mt, -1)
+
+    (c0, s0), (c1, s1) = run(M), run(tall)
+    np.testing.assert_array_equal(c0, c1[:M])
+    if nw >= 0:
+        np.testing.assert_array_equal(s0[:M // 128], s1[:M // 128])
