@@ -36,6 +36,10 @@ constexpr int kTile = kMssTile;    // output samples owned by a workgroup
 constexpr int kHalo = kMssHalo;    // largest N - 1
 constexpr int kAcc = kMssAcc;
 constexpr int kThreads = 256;
+// Tiles up to which a workgroup takes two groups at a time: those that have a
+// CU each.  256 tiles of six sizes 107 us against 154 a group at a time; 264
+// would take two rounds, 214, where two one-group workgroups share a CU in 174.
+constexpr int kPairTiles = 256;
 constexpr int kMaxSizes = 8;
 constexpr float kLogEps = 1e-8f;   // DGenSpectralConfig.logMagnitudeEpsilon (GradientConfig.swift:38)
 constexpr float kMagEps = 1e-8f;   // safeMag = max(mag, 1e-8) (Emit+SpectralLoss.swift:1005-1006)
@@ -62,6 +66,12 @@ __device__ __forceinline__ float hw_sqrt(float v) { return __builtin_amdgcn_sqrt
 __device__ __forceinline__ float hw_log(float v) { return __builtin_amdgcn_logf(v) * 0.69314718055994531f; }
 __device__ __forceinline__ float hw_rcp(float v) { return __builtin_amdgcn_rcpf(v); }
 
+// fused by name: left to the compiler, the products of a conditional add are
+// formed before its branch and rounded on their own
+__device__ __forceinline__ float2 fma2(c2 v, float2 h, float2 a) {
+  return {__builtin_fmaf(v.x, h.x, a.x), __builtin_fmaf(v.y, h.y, a.y)};
+}
+
 // LDS of the launch (every size runs in it, one after the other).
 // The tile accumulator holds dx of samples [a - kHalo, a + kTile) (whole
 // 64-sample blocks), stored swizzled: sample i lives at
@@ -75,15 +85,16 @@ __device__ __forceinline__ float hw_rcp(float v) { return __builtin_amdgcn_rcpf(
 // padding.
 __device__ __forceinline__ int accp(int i) { return i ^ (((i >> 6) & 7) << 3); }
 
+template <int HV>
 struct MssLds {
   static constexpr int kAccN = kAcc + 1;  // 64-sample blocks
   float acc[kAccN];
-  c2 buf[2048];                    // FFT slots: (4096/N windows) x (N/2), swizzled
-  c2 aux[2048];                    // second signal's spectrum / gradient spectrum
-  float red[kThreads / 64][2];
+  c2 buf[HV][2048];                // FFT slots: (4096/N windows) x (N/2), swizzled
+  c2 aux[HV][2048];                // second signal's spectrum / gradient spectrum
+  float red[HV * kThreads / 64][2];
   c2 tw[1024];                     // this size's exp(-2 pi i k / N), k < N/2, correctly rounded
 };
-static_assert(MssLds::kAccN % 64 == 0, "the accumulator swizzle works on whole 64-sample blocks");
+static_assert(MssLds<1>::kAccN % 64 == 0, "the accumulator swizzle works on whole 64-sample blocks");
 
 // One FFT size: 4 groups of 4096/N windows, windows in a group 4 hops apart.
 // tid: the thread's index, opaque to the optimiser in each call (else every
@@ -91,8 +102,11 @@ static_assert(MssLds::kAccN % 64 == 0, "the accumulator swizzle works on whole 6
 // and held in registers together)
 // GEN: the generic bin arithmetic (a.mode's L1/L2 terms and smooth log
 // magnitude); otherwise the trainer's L1 magnitude and log(mag + eps) terms
-template <int LOGN, bool GEN>
-__device__ __forceinline__ void mss_size(const MssArgs& a, MssLds& L, int si, int b, int tile, int tid) {
+// HV: groups transformed side by side, each by kThreads threads (half) on
+// buffers of its own; they add to the accumulator one after the other, so
+// every sample is summed in the same order.
+template <int LOGN, bool GEN, int HV>
+__device__ __forceinline__ void mss_size(const MssArgs& a, MssLds<HV>& L, int si, int b, int tile, int tid, int half) {
   constexpr int N = 1 << LOGN, M = N / 2, LOGM = LOGN - 1, H = N / 4, P = M / 8, W = kThreads / P;
   static_assert(W * M == 2048, "window slots must fill the FFT buffer");
   // accumulator index of sample t: t - (a0 - kHalo); for an output pair of a
@@ -104,8 +118,8 @@ __device__ __forceinline__ void mss_size(const MssArgs& a, MssLds& L, int si, in
   // consecutive groups overlap) and for the cross-wave loss sums (P > 64)
   constexpr bool WL = P <= 64;
   const int slot = tid / P, j = tid % P;
-  const SwzBuf buf(L.buf, slot * M);
-  const SwzBuf spec(L.aux, slot * M);
+  const SwzBuf buf(L.buf[half], slot * M);
+  const SwzBuf spec(L.aux[half], slot * M);
   const int sj = buf.part(j);  // spec.part(j) too
   const int a0 = tile * kTile;
   const int nwin = (a.T + H - 1) / H;
@@ -140,7 +154,7 @@ __device__ __forceinline__ void mss_size(const MssArgs& a, MssLds& L, int si, in
     }
 #pragma unroll
     for (int q = 0; q < TP; ++q)
-      if (tid + q * kThreads < M) L.tw[tid + q * kThreads] = c2{cv[q], -sv[q]};
+      if (half == 0 && tid + q * kThreads < M) L.tw[tid + q * kThreads] = c2{cv[q], -sv[q]};
   }
   lds_barrier();
   const RegTwiddle<LOGM> tw(TableTwiddle{L.tw, M}, j);
@@ -178,9 +192,9 @@ __device__ __forceinline__ void mss_size(const MssArgs& a, MssLds& L, int si, in
       }
     }
   };
-  fetch(0);
+  fetch(half);
 #pragma unroll 1
-  for (int g = 0; g < 4; ++g) {
+  for (int g = half; g < 4; g += HV) {
     const int w = a0 / H + g + 4 * slot;
     const bool live = w < nwin && w * H < a0 + kTile;
     const int f = w * H;
@@ -202,7 +216,7 @@ __device__ __forceinline__ void mss_size(const MssArgs& a, MssLds& L, int si, in
       fft_store<LOGM>(buf, j, v);
       lds_sync<WL>();
     }
-    if (g + 1 < 4) fetch(g + 1);  // overlaps the bins and the inverse transform
+    if (g + HV < 4) fetch(g + HV);  // overlaps the bins and the inverse transform
     // ---- bins: pair (k, M-k) for k = 0..M/2 gives every bin 0..N/2; each
     //      thread owns the pairs k = j + i*P (i < NB)
     float lin = 0.f, lg = 0.f;
@@ -308,7 +322,7 @@ __device__ __forceinline__ void mss_size(const MssArgs& a, MssLds& L, int si, in
       lg += __shfl_xor(lg, off, 64);
     }
     if (P > 64) {
-      const int wv = tid >> 6;
+      const int wv = half * (kThreads / 64) + (tid >> 6);
       if ((tid & 63) == 0) {
         L.red[wv][0] = lin;
         L.red[wv][1] = lg;
@@ -318,7 +332,7 @@ __device__ __forceinline__ void mss_size(const MssArgs& a, MssLds& L, int si, in
     if (j == 0 && live) {
       float sl = lin, sg = lg;
       if (P > 64) {
-        const int w0 = (slot * P) >> 6;
+        const int w0 = half * (kThreads / 64) + ((slot * P) >> 6);
         sl = 0.f;
         sg = 0.f;
         for (int q = 0; q < P / 64; ++q) {
@@ -340,71 +354,86 @@ __device__ __forceinline__ void mss_size(const MssArgs& a, MssLds& L, int si, in
     // pair is one 8-byte LDS access.  Pairs outside the tile's range read a
     // clamped element and are not written; a pair with one sample outside
     // [0, T) writes only the other.
-    if (live && s0 >= 0 && s0 + N <= a.T) {
-      // the whole window inside [0, T): every pair is written
-      float2 ac[8];
-      int ai[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        ai[e] = accp(f - a0 + kOff + 2 * op[e]);
-        ac[e] = *reinterpret_cast<const float2*>(&L.acc[ai[e]]);
+    auto overlap_add = [&]() {
+      if (live && s0 >= 0 && s0 + N <= a.T) {
+        // the whole window inside [0, T): every pair is written
+        float2 ac[8];
+        int ai[8];
+  #pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          ai[e] = accp(f - a0 + kOff + 2 * op[e]);
+          ac[e] = *reinterpret_cast<const float2*>(&L.acc[ai[e]]);
+        }
+  #pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float2 h = hout[e];
+          *reinterpret_cast<float2*>(&L.acc[ai[e]]) = fma2(v[e], h, ac[e]);
+        }
+      } else {
+        constexpr int kAccN = MssLds<HV>::kAccN;
+        float2 ac[8];
+        int ai[8];
+        bool a0w[8], a1w[8];
+  #pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int t = s0 + 2 * op[e];
+          a0w[e] = live && t >= 0 && t < a.T;
+          a1w[e] = live && t + 1 >= 0 && t + 1 < a.T;
+          ai[e] = accp(min(max(t - (a0 - kHalo), 0), kAccN - 2));
+          ac[e] = *reinterpret_cast<const float2*>(&L.acc[ai[e]]);
+        }
+  #pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float2 h = hout[e];
+          const float2 r = fma2(v[e], h, ac[e]);
+          if (a0w[e] && a1w[e]) *reinterpret_cast<float2*>(&L.acc[ai[e]]) = r;
+          else if (a0w[e]) L.acc[ai[e]] = r.x;
+          else if (a1w[e]) L.acc[ai[e] + 1] = r.y;
+        }
       }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float2 h = hout[e];
-        *reinterpret_cast<float2*>(&L.acc[ai[e]]) = float2{ac[e].x + v[e].x * h.x, ac[e].y + v[e].y * h.y};
-      }
+    };
+    // every wave's overlap-add of group g lands before any of group g + 1
+    if constexpr (HV == 1) {
+      overlap_add();
+      lds_barrier();
     } else {
-      constexpr int kAccN = MssLds::kAccN;
-      float2 ac[8];
-      int ai[8];
-      bool a0w[8], a1w[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int t = s0 + 2 * op[e];
-        a0w[e] = live && t >= 0 && t < a.T;
-        a1w[e] = live && t + 1 >= 0 && t + 1 < a.T;
-        ai[e] = accp(min(max(t - (a0 - kHalo), 0), kAccN - 2));
-        ac[e] = *reinterpret_cast<const float2*>(&L.acc[ai[e]]);
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float2 h = hout[e];
-        const float2 r = {ac[e].x + v[e].x * h.x, ac[e].y + v[e].y * h.y};
-        if (a0w[e] && a1w[e]) *reinterpret_cast<float2*>(&L.acc[ai[e]]) = r;
-        else if (a0w[e]) L.acc[ai[e]] = r.x;
-        else if (a1w[e]) L.acc[ai[e] + 1] = r.y;
+#pragma unroll 1
+      for (int h = 0; h < HV; ++h) {
+        if (half == h) overlap_add();
+        lds_barrier();
       }
     }
-    // every wave's overlap-add of group g lands before any of group g + 1
-    lds_barrier();
   }
 }
 
 // All sizes in one launch, in the op's size order: the tile accumulator
 // stays in LDS from the first size to the last and is written to the tile
 // partials once.
-template <bool GEN>
-__global__ __launch_bounds__(kThreads) void k_mss(MssArgs a) {
-  extern __shared__ float4 smem4[];
-  MssLds& L = *reinterpret_cast<MssLds*>(smem4);
+// HV = 2 (tiles for less than the chip): a workgroup alone on its CU leaves the
+// SIMDs waiting between its four waves' dependent steps, so eight waves run
+// two groups of every four at a time: a tile of six sizes 152 -> 101 us alone.
+template <bool GEN, int HV>
+__global__ __launch_bounds__(HV* kThreads) void k_mss(MssArgs a) {
+  __shared__ float4 smem4[(sizeof(MssLds<HV>) + 15) / 16];
+  MssLds<HV>& L = *reinterpret_cast<MssLds<HV>*>(smem4);
   const int tile = blockIdx.x, b = blockIdx.y;
-  for (int i = threadIdx.x; i < MssLds::kAccN; i += kThreads) L.acc[i] = 0.f;
+  const int half = HV == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads);
+  for (int i = threadIdx.x; i < MssLds<HV>::kAccN; i += HV * kThreads) L.acc[i] = 0.f;
   lds_barrier();
   for (int s = 0; s < a.nsizes; ++s) {
-    int tid = threadIdx.x;
+    int tid = threadIdx.x % kThreads;
     asm volatile("" : "+v"(tid));
     switch (a.logn[s]) {
-      case 6: mss_size<6, GEN>(a, L, s, b, tile, tid); break;
-      case 7: mss_size<7, GEN>(a, L, s, b, tile, tid); break;
-      case 8: mss_size<8, GEN>(a, L, s, b, tile, tid); break;
-      case 9: mss_size<9, GEN>(a, L, s, b, tile, tid); break;
-      case 10: mss_size<10, GEN>(a, L, s, b, tile, tid); break;
-      default: mss_size<11, GEN>(a, L, s, b, tile, tid); break;
+      case 6: mss_size<6, GEN, HV>(a, L, s, b, tile, tid, half); break;
+      case 7: mss_size<7, GEN, HV>(a, L, s, b, tile, tid, half); break;
+      case 8: mss_size<8, GEN, HV>(a, L, s, b, tile, tid, half); break;
+      case 9: mss_size<9, GEN, HV>(a, L, s, b, tile, tid, half); break;
+      case 10: mss_size<10, GEN, HV>(a, L, s, b, tile, tid, half); break;
+      default: mss_size<11, GEN, HV>(a, L, s, b, tile, tid, half); break;
     }
   }
   float* part = a.part + ((size_t)b * a.ntiles + tile) * kAcc;
-  for (int i = threadIdx.x; i < kAcc; i += kThreads) part[i] = L.acc[accp(i)];
+  for (int i = threadIdx.x; i < kAcc; i += HV * kThreads) part[i] = L.acc[accp(i)];
 }
 
 int launch_spectral_loss(const Launch& L, const dgen_hip_op& op) {
@@ -449,10 +478,10 @@ int launch_spectral_loss(const Launch& L, const dgen_hip_op& op) {
   a.gg = op.farg[1];
   a.mode = (int)mode;
   const dim3 grid((unsigned)ntiles, (unsigned)B);
-  if (mode)
-    hipLaunchKernelGGL(k_mss<true>, grid, dim3(kThreads), sizeof(MssLds), L.stream, a);
-  else
-    hipLaunchKernelGGL(k_mss<false>, grid, dim3(kThreads), sizeof(MssLds), L.stream, a);
+  const bool pair = ntiles * B <= kPairTiles;
+  const dim3 block(pair ? 2 * kThreads : kThreads);
+  auto* kernel = mode ? (pair ? k_mss<true, 2> : k_mss<true, 1>) : (pair ? k_mss<false, 2> : k_mss<false, 1>);
+  hipLaunchKernelGGL(kernel, grid, block, 0, L.stream, a);
   DGEN_LAUNCH_CHECK("k_mss");
   return 0;
 }
