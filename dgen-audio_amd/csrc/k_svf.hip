@@ -652,11 +652,22 @@ __global__ __launch_bounds__(64 * kRepairWaves) void k_svf_repair(SpecArgs a, co
   if (wave > 0) return;
 #pragma unroll
   for (int w = 0; w < kRepairWaves; ++w) bad = min(bad, s_bad[w][lane]);
-  if (kk >= B || bad >= a.C) return;
+  // the wave steps the spans together, so that a span's rows stay at uniform
+  // addresses; a lane joins in at its own first bad one
+  int first = kk < B ? bad : a.C;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) first = min(first, __shfl_xor(first, off, 64));
+  first = __builtin_amdgcn_readfirstlane(first);
+  if (first >= a.C || kk >= B) return;
   const float kd = 1.0f / a.prm[B + k], ks = a.prm[2 * B + k];
-  size_t o = (size_t)bad * 2 * B + k;
-  float c1 = end[o - 2 * (size_t)B], c2 = end[o - (size_t)B];
-  for (int c = bad; c < a.C; ++c, o += 2 * (size_t)B) {
+  float c1 = 0.0f, c2 = 0.0f;
+  for (int c = first; c < a.C; ++c) {
+    const size_t o = (size_t)c * 2 * B + k;
+    if (c < bad) continue;
+    if (c == bad) {
+      c1 = end[o - 2 * (size_t)B];
+      c2 = end[o - (size_t)B];
+    }
     if (same_bits(c1, a.start[o]) && same_bits(c2, a.start[o + B])) {
       c1 = end[o];
       c2 = end[o + B];
