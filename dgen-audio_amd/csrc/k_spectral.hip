@@ -11,7 +11,7 @@
 // zero) goes through an unnormalised inverse transform whose real part,
 // times the window, is added to dx over the window's samples.
 //
-// Work decomposition (one workgroup = 256 threads):
+// Work decomposition (one workgroup = 256 threads, twice that for few tiles):
 // - the workgroup owns an output tile [a, a+4096) of one batch lane and all
 //   windows whose hop frame lies in it, for every size;
 // - a real N-point transform is an N/2-point complex Stockham FFT of
