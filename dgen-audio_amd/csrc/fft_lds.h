@@ -80,8 +80,9 @@ __device__ __forceinline__ c2 cis(float rev) { return {__builtin_amdgcn_cosf(rev
 
 // Twiddle sources of the passes.  A pass of radix R and span NS multiplies
 // input r of butterfly k by W^(r k) with W = exp(-+2 pi i / (NS R)).
-// - HwTwiddle: W^1 from the hardware sin/cos (about 2 ulp), higher powers by
-//   complex products (up to six for radix 8);
+// - HwRegTwiddle (below): W^1 from the hardware sin/cos (about 2 ulp), higher
+//   powers by complex products (up to six for radix 8), formed once into
+//   registers for one thread's butterflies;
 // - TableTwiddle: every power read from a table of correctly rounded values
 //   t[i] = exp(-2 pi i i / N), i < N/2 = M (the last radix-2 stage's row of
 //   the reference's Float twiddle table, HigherOps.swift:84-91), as
@@ -90,11 +91,7 @@ __device__ __forceinline__ c2 cis(float rev) { return {__builtin_amdgcn_cosf(rev
 //   log-magnitude gradient amplifies it), so the spectral loss uses tables;
 // - RegTwiddle (below): the same table values for one thread's butterflies,
 //   read once into registers.
-struct HwTwiddle {
-  static constexpr bool kTable = false;
-};
 struct TableTwiddle {
-  static constexpr bool kTable = true;
   const c2* t;  // M values, in LDS
   int m;
   // W_M^e for 0 <= e < M (forward sign)
@@ -169,7 +166,6 @@ __host__ __device__ constexpr int ilog2c(int n) { return n <= 1 ? 0 : 1 + ilog2c
 // a pass share their index k (and twiddles) when NS divides M/8.
 template <int LOGM>
 struct RegTwiddle {
-  static constexpr bool kTable = true;
   static constexpr int M = 1 << LOGM, NP = pass_count(LOGM);
   template <int R, int NS>
   static constexpr int nu() { return (M / 8) % NS == 0 ? 1 : 8 / R; }
@@ -195,12 +191,10 @@ struct RegTwiddle {
   }
 };
 
-// HwTwiddle's values for one thread's butterflies, in registers: the same
-// hardware sin/cos and products, evaluated once per kernel instead of in every
+// Hardware sin/cos and products, evaluated once per kernel instead of in every
 // transform (the inverse's are the conjugates, bit for bit).
 template <int LOGM>
 struct HwRegTwiddle {
-  static constexpr bool kTable = true;
   static constexpr int M = 1 << LOGM, NP = pass_count(LOGM);
   template <int R, int NS>
   static constexpr int nu() { return (M / 8) % NS == 0 ? 1 : 8 / R; }
@@ -279,26 +273,15 @@ __device__ __forceinline__ void pass_store(const SwzBuf& buf, int j, const c2* v
 // butterfly k: w[r] *= W^(r k).
 template <int M, int R, int NS, bool INV, class TW>
 __device__ __forceinline__ void twiddle(c2* w, int u, int k, const TW& tw) {
-  if constexpr (TW::kTable) {
 #pragma unroll
-    for (int r = 1; r < R; ++r) {
-      const c2 t = tw.template pass_tw<M, R, NS>(u, r, k);
-      w[r] = cmul(w[r], INV ? cconj(t) : t);
-    }
-  } else {
-    const float rev = (INV ? 1.0f : -1.0f) * (float)k / (float)(NS * R);
-    const c2 t1 = cis(rev);
-    c2 t = t1;
-#pragma unroll
-    for (int r = 1; r < R; ++r) {
-      w[r] = cmul(w[r], t);
-      if (r + 1 < R) t = cmul(t, t1);
-    }
+  for (int r = 1; r < R; ++r) {
+    const c2 t = tw.template pass_tw<M, R, NS>(u, r, k);
+    w[r] = cmul(w[r], INV ? cconj(t) : t);
   }
 }
 
-template <int M, int R, int NS, bool INV, class TW = HwTwiddle>
-__device__ __forceinline__ void pass_compute(c2* v, int j, int* outpos, const TW& tw = TW{}) {
+template <int M, int R, int NS, bool INV, class TW>
+__device__ __forceinline__ void pass_compute(c2* v, int j, int* outpos, const TW& tw) {
   constexpr int BPT = 8 / R;
 #pragma unroll
   for (int u = 0; u < BPT; ++u) {
@@ -312,8 +295,8 @@ __device__ __forceinline__ void pass_compute(c2* v, int j, int* outpos, const TW
 
 // Middle passes 1 .. npass-2 in LDS (in place; a sync separates each pass's
 // reads from its writes).
-template <int LOGM, int P, bool INV, bool WAVE = false, class TW = HwTwiddle>
-__device__ __forceinline__ void mid_passes(const SwzBuf& buf, int j, int sj, c2* v, const TW& tw = TW{}) {
+template <int LOGM, int P, bool INV, bool WAVE = false, class TW>
+__device__ __forceinline__ void mid_passes(const SwzBuf& buf, int j, int sj, c2* v, const TW& tw) {
   constexpr int M = 1 << LOGM;
   if constexpr (P < pass_count(LOGM) - 1) {
     constexpr int R = pass_radix(LOGM, P), NS = pass_span(LOGM, P);
@@ -342,8 +325,8 @@ __device__ __forceinline__ void fft_store(const SwzBuf& buf, int j, const c2* v)
 // Full M-point FFT: v holds the first pass's inputs (v[e] = input at
 // in_pos of pass 0); on return v holds the last pass's outputs at positions
 // op[e].  Uses buf (M complex, this window's slot) between passes.
-template <int LOGM, bool INV, bool WAVE = false, class TW = HwTwiddle>
-__device__ __forceinline__ void fft(const SwzBuf& buf, int j, c2* v, int* op, const TW& tw = TW{}) {
+template <int LOGM, bool INV, bool WAVE = false, class TW>
+__device__ __forceinline__ void fft(const SwzBuf& buf, int j, c2* v, int* op, const TW& tw) {
   constexpr int M = 1 << LOGM;
   constexpr int NP = pass_count(LOGM);
   constexpr int R0 = pass_radix(LOGM, 0);
@@ -365,8 +348,8 @@ __device__ __forceinline__ void fft(const SwzBuf& buf, int j, c2* v, int* op, co
 // positions and LDS round trip serve both, and the two butterflies give the
 // scheduler independent work.  Each signal's arithmetic is exactly that of
 // fft().
-template <int M, int R, int NS, bool INV, class TW = HwTwiddle>
-__device__ __forceinline__ void pass_compute2(c2* va, c2* vb, int j, int* outpos, const TW& tw = TW{}) {
+template <int M, int R, int NS, bool INV, class TW>
+__device__ __forceinline__ void pass_compute2(c2* va, c2* vb, int j, int* outpos, const TW& tw) {
   constexpr int BPT = 8 / R;
 #pragma unroll
   for (int u = 0; u < BPT; ++u) {
@@ -374,24 +357,12 @@ __device__ __forceinline__ void pass_compute2(c2* va, c2* vb, int j, int* outpos
     c2* wa = va + u * R;
     c2* wb = vb + u * R;
     if (NS > 1) {
-      if constexpr (TW::kTable) {
 #pragma unroll
-        for (int r = 1; r < R; ++r) {
-          const c2 t0 = tw.template pass_tw<M, R, NS>(u, r, k);
-          const c2 t = INV ? cconj(t0) : t0;
-          wa[r] = cmul(wa[r], t);
-          wb[r] = cmul(wb[r], t);
-        }
-      } else {
-        const float rev = (INV ? 1.0f : -1.0f) * (float)k / (float)(NS * R);
-        const c2 t1 = cis(rev);
-        c2 t = t1;
-#pragma unroll
-        for (int r = 1; r < R; ++r) {
-          wa[r] = cmul(wa[r], t);
-          wb[r] = cmul(wb[r], t);
-          if (r + 1 < R) t = cmul(t, t1);
-        }
+      for (int r = 1; r < R; ++r) {
+        const c2 t0 = tw.template pass_tw<M, R, NS>(u, r, k);
+        const c2 t = INV ? cconj(t0) : t0;
+        wa[r] = cmul(wa[r], t);
+        wb[r] = cmul(wb[r], t);
       }
     }
     dftR<R, INV>(wa);
@@ -400,9 +371,9 @@ __device__ __forceinline__ void pass_compute2(c2* va, c2* vb, int j, int* outpos
   pass_positions<M, R, NS>(j, outpos);
 }
 
-template <int LOGM, int P, bool INV, bool WAVE, class TW = HwTwiddle>
+template <int LOGM, int P, bool INV, bool WAVE, class TW>
 __device__ __forceinline__ void mid_passes2(const SwzBuf& bufa, const SwzBuf& bufb, int j, int sj, c2* va, c2* vb,
-                                            const TW& tw = TW{}) {
+                                            const TW& tw) {
   constexpr int M = 1 << LOGM;
   if constexpr (P < pass_count(LOGM) - 1) {
     constexpr int R = pass_radix(LOGM, P), NS = pass_span(LOGM, P);
@@ -421,9 +392,9 @@ __device__ __forceinline__ void mid_passes2(const SwzBuf& bufa, const SwzBuf& bu
 // fft() of two signals at once (bufa and bufb: the same slot of two
 // buffers): on return va / vb hold their last pass's outputs at positions
 // op[e].
-template <int LOGM, bool INV, bool WAVE = false, class TW = HwTwiddle>
+template <int LOGM, bool INV, bool WAVE = false, class TW>
 __device__ __forceinline__ void fft2(const SwzBuf& bufa, const SwzBuf& bufb, int j, c2* va, c2* vb, int* op,
-                                     const TW& tw = TW{}) {
+                                     const TW& tw) {
   constexpr int M = 1 << LOGM;
   constexpr int NP = pass_count(LOGM);
   constexpr int R0 = pass_radix(LOGM, 0);
