@@ -14,6 +14,12 @@ from .program import Program
 from .workloads import (BiquadConfig, HarmonicConfig, MembraneConfig, OscBankConfig, StftConfig, SvfConfig,
                         SweptPhasorConfig)
 
+
+class DefaultChunk(int):
+    """A scan's chunk length as the builders choose it, so that they may
+    shorten it (`_scan_chunk`); a plain int is a caller's and is kept."""
+
+
 SEG = 64          # frames per synth segment (checkpoint spacing)
 SLOTS = 4         # control rows a segment may touch
 ROW_ENTRIES = 16  # (segment, slot) entries per control row (kRowEntries)
@@ -26,8 +32,8 @@ GEMM_TILE_M = 128  # output rows per GEMM workgroup tile (k_gemm.hip BM)
 GEMM_SMALL_TILES = 128  # 128 x 128 tiles up to which a split-bf16 GEMM splits its own operands (k_gemm.hip kSmTiles)
 SPLITK_ROWS_HEADS = 256  # the heads' weight gradient has one 128-wide column tile: split finer to fill the chip
 MSS_TILE = 4096     # output samples per spectral-loss workgroup
-BQ_CHUNK = 512      # frames per biquad scan chunk (512 measured fastest of 128..1024)
-SVF_CHUNK = 256     # frames per SVF scan chunk
+BQ_CHUNK = DefaultChunk(512)   # frames per biquad scan chunk (512 measured fastest of 128..1024)
+SVF_CHUNK = DefaultChunk(256)  # frames per SVF scan chunk
 SCAN_WAVES = 2048   # waves (64 lanes x one chunk) a filter scan's passes should have: two per SIMD
 STFT_TILE = 8192    # largest output tile of an STFT forward workgroup
 STFT_GROUPS = 512   # workgroups an STFT pass is split into if need be (two per CU)
@@ -451,16 +457,18 @@ class HarmonicSession:
 
 # ------------------------------------------------------------------ config 4
 def _scan_chunk(B: int, T: int, chunk: int) -> int:
-    """Frames per chunk of a filter bank's scans: `chunk`, halved (to no less
-    than 32, in whole thirty-twos) while the lanes and chunks make fewer than
-    SCAN_WAVES waves.  A pass lasts as long as one chunk's frames in sequence
+    """Frames per chunk of a filter bank's scans: `chunk`, a default one halved
+    (to no less than 32, in whole thirty-twos) while the lanes and chunks make
+    fewer than SCAN_WAVES waves.  A pass lasts as long as one chunk's frames in sequence
     (~0.25 us each), so few lanes or a short signal want shorter chunks; with
     the chip full, shorter ones only add chunk maps to the carry.  Steps
     measured: biquad 12 lanes x 8192 frames 488 us at 512, 134 at 32, 137 at
     16; linear SVF 70 x 30001 368 us at 256, 216 at 64, 197 at 32, 236 at 16;
     saturating SVF 256 x 65536 814 us at 256, 755 at 128, 765 at 64; biquad 256
     x 2^18 605 us at 512 (kept), 624 at 256, 678 at 128."""
-    L, groups = chunk, (B + 63) // 64
+    L, groups = int(chunk), (B + 63) // 64
+    if not isinstance(chunk, DefaultChunk):
+        return L
     while L % 64 == 0 and groups * ((T + L - 1) // L) < SCAN_WAVES:
         L //= 2
     return L
@@ -485,7 +493,7 @@ def biquad_program(cfg: BiquadConfig, train: bool = True, optimizer: bool = True
     B, T, L = cfg.B, cfg.T, int(chunk)
     if L <= 0:
         raise ValueError("chunk length must be positive")
-    L = _scan_chunk(B, T, L)
+    L = _scan_chunk(B, T, chunk)
     C = (T + L - 1) // L
     f4 = 4.0
     p = Program(max_frames=T)
@@ -634,7 +642,7 @@ def svf_program(cfg: SvfConfig, train: bool = True, optimizer: bool = True, satu
     if L <= 0:
         raise ValueError("chunk length must be positive")
     P = 3 if sat else 2
-    L = _scan_chunk(B, T, L)
+    L = _scan_chunk(B, T, chunk)
     C = (T + L - 1) // L
     f4 = 4.0
     n = float(T * B)
