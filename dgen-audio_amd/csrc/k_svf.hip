@@ -521,11 +521,13 @@ __device__ __forceinline__ void svf_span(const float* __restrict__ x, const floa
   const Rows ra = T3 ? rows_at(cells, n0, cnt, B) : rx, rb = T3 ? rows_at(cells, (size_t)T + n0, cnt, B) : rx;
   const int col = k * (int)sizeof(float), pitch = B * (int)sizeof(float);
   float cx[kSpecG], cg[kSpecG], ct[kSpecG];
-  // (rows past the end read as 0)
-  auto load = [&](int i, float (&vx)[kSpecG], float (&vg)[kSpecG], float (&vt)[kSpecG]) {
+  // (a uniform offset is not certain to count in the buffer's bounds check, so
+  // rows past the end are kept away from by index: the main loop's loads lie
+  // inside, `edge` ones read the last row again)
+  auto load = [&](auto edge, int i, float (&vx)[kSpecG], float (&vg)[kSpecG], float (&vt)[kSpecG]) {
 #pragma unroll
     for (int j = 0; j < kSpecG; ++j) {
-      const int r = (i + j) * pitch;
+      const int r = (edge() ? min(i + j, cnt - 1) : i + j) * pitch;
       vx[j] = row_load(rx, col, r);
       vg[j] = row_load(rg, col, r);
       if constexpr (T3) vt[j] = row_load(rt, col, r);
@@ -567,18 +569,21 @@ __device__ __forceinline__ void svf_span(const float* __restrict__ x, const floa
       left = L;
     }
   };
-  load(0, cx, cg, ct);
+  const std::false_type in;
+  const std::true_type edge;
+  load(edge, 0, cx, cg, ct);
   float nx[kSpecG], ng[kSpecG], nt[kSpecG];
-  while (i + 2 * kSpecG <= cnt) {
-    load(i + kSpecG, nx, ng, nt);
+  while (i + 3 * kSpecG <= cnt) {
+    load(in, i + kSpecG, nx, ng, nt);
     __builtin_amdgcn_sched_barrier(0);
     group(cx, cg, ct);
-    load(i + kSpecG, cx, cg, ct);
+    load(in, i + kSpecG, cx, cg, ct);
     __builtin_amdgcn_sched_barrier(0);
     group(nx, ng, nt);
   }
-  if (i + kSpecG <= cnt) {
-    load(i + kSpecG, nx, ng, nt);
+  while (i + kSpecG <= cnt) {  // at most twice
+    load(edge, i + kSpecG, nx, ng, nt);
+    __builtin_amdgcn_sched_barrier(0);
     group(cx, cg, ct);
 #pragma unroll
     for (int j = 0; j < kSpecG; ++j) {
