@@ -626,9 +626,9 @@ constexpr int kSbForm = kThreads - 64;
 static_assert(kSbLanes * kSbF % kSbForm == 0, "whole elements per forming thread");
 
 template <bool MOD>
-__global__ __launch_bounds__(kThreads) void k_stream_bq(const float* __restrict__ x, const float* __restrict__ mod,
+__global__ __launch_bounds__(kThreads) void k_stream_bq(const float* x, const float* __restrict__ mod,
                                                         const float* __restrict__ prm, float* __restrict__ state,
-                                                        float* __restrict__ y, int B, int T, int reset) {
+                                                        float* y, int B, int T, int reset) {
   __shared__ __align__(16) float sF[2][kSbLanes][kSbLd], s1[2][kSbLanes][kSbLd], s2[2][kSbLanes][kSbLd];
   __shared__ __align__(16) float sy[2][kSbLanes][kSbLd];
   const int ntile = (T + kSbF - 1) / kSbF, k0 = blockIdx.x * kSbLanes;
@@ -682,6 +682,13 @@ __global__ __launch_bounds__(kThreads) void k_stream_bq(const float* __restrict_
     y1 = state[2 * B + k];
     y2 = state[3 * B + k];
   }
+  // the input history it leaves, read before any frame is stored: y may be x
+  // itself (a tile is stored only after the next one's x has been read)
+  float e1 = 0.0f, e2 = h1;
+  if (chain) {
+    e1 = x[(size_t)(T - 1) * B + k];
+    if (T >= 2) e2 = x[(size_t)(T - 2) * B + k];
+  }
   if (wave > 0) form(0);
   __syncthreads();
   for (int t = 0; t < ntile; ++t) {
@@ -717,8 +724,8 @@ __global__ __launch_bounds__(kThreads) void k_stream_bq(const float* __restrict_
   }
   if (wave > 0) store(ntile - 1);
   if (chain) {
-    state[k] = x[(size_t)(T - 1) * B + k];
-    state[B + k] = T >= 2 ? x[(size_t)(T - 2) * B + k] : h1;
+    state[k] = e1;
+    state[B + k] = e2;
     state[2 * B + k] = y1;
     state[3 * B + k] = y2;
   }

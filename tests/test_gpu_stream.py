@@ -163,3 +163,29 @@ def test_biquad_blocks_over_tile_edges(B, sizes):
     ref = O.biquad_stream(x, mod, p[:B], p[B:], np.zeros((B, 4), np.float32))
     ref64 = O.biquad_fwd(x, mod, p[:B].astype(np.float64), p[B:].astype(np.float64), prec="f64")
     assert np.abs(one - ref64).max() <= 2.0 * np.abs(ref - ref64).max() + 1e-7
+
+
+@pytest.mark.parametrize("B,sizes", [(3, [1, 2, 97]), (9, [96, 95, 300])])
+def test_biquad_blocks_in_place(B, sizes):
+    """An op whose output cell is its input cell gives the samples and the
+    carried history of one with cells of their own, bit for bit."""
+    T = sum(sizes)
+    cfg = BiquadConfig(B=B, T=T)
+    x, mod = cfg.inputs(), cfg.modulation()
+    rt = bq_runtime(cfg)
+    try:
+        want = bq_calls(rt, x, mod, sizes)
+    finally:
+        rt.close()
+    prog = stream_biquad_program(cfg)
+    op = prog.ops[prog.find("stream_biquad")]
+    op.arg[4] = op.arg[0]
+    ins, outs = prog.meta["ports"]
+    print(f"streaming biquad bank in place B={B} blocks {sizes}", flush=True)
+    rt = HIPLazyRuntime(prog, 0)
+    try:
+        rt.write("params", cfg.params())
+        rt.setProcessPorts(ins, [("x", k, stride) for _, k, stride in outs])
+        np.testing.assert_array_equal(bq_calls(rt, x, mod, sizes), want)
+    finally:
+        rt.close()
