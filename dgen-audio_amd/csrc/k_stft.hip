@@ -159,7 +159,9 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
   auto add = [&](int w, const c2 (&v)[8], const int (&op)[8]) {
     const int h = w * H, o = h - a0;
     const bool whole = w <= w_hi && o >= 0 && h + N <= a1;
-    if (__ballot(!whole) == 0 && H % 2 == 0) {
+    // pairs of the tile are 8-byte aligned where o is even: even hops from an
+    // even tile start
+    if (__ballot(!whole) == 0 && (H | a0) % 2 == 0) {
 #pragma unroll
       for (int e0 = 0; e0 < 8; e0 += 4) {
         float2 t[4];

@@ -150,7 +150,7 @@ def test_full_configuration_matches_oracle(gpu):
 @pytest.mark.parametrize("S,T,N,H", [(2, 9001, 64, 16), (1, 5000, 64, 1), (2, 9001, 128, 33), (3, 20000, 256, 64),
                                      (1, 20003, 512, 171), (2, 30001, 1024, 256), (1, 9000, 1024, 100),
                                      (2, 20000, 2048, 512), (1, 9000, 2048, 2048)])
-@pytest.mark.parametrize("tile,rounds", [(256, 1), (512, 2), (1280, 3), (8192, 8)])
+@pytest.mark.parametrize("tile,rounds", [(256, 1), (257, 1), (512, 2), (1280, 3), (1281, 3), (8192, 8)])
 def test_tiles_and_rounds_agree_with_the_oracle(gpu, S, T, N, H, tile, rounds):
     """Output tiles and gradient runs of any length: windows added in phases
     (tiles shorter than the windows of a round span) or a run per slot, odd
