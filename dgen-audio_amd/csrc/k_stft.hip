@@ -21,8 +21,9 @@
 // per complex value.  W windows (one per M/8-thread slot) are transformed at
 // once, and each slot adds its outputs from registers to the tile accumulator
 // (read, add, write; windows added at the same time do not overlap, so the
-// sum is atomic-free and its order fixed).  The tile then yields y,
-// dL/dy = 2 (y - x)/T and its share of the loss sum (y - x)^2 / T.
+// sum is atomic-free, in an order that neither tile nor batch changes).  The
+// tile then yields y, dL/dy = 2 (y - x)/T and its share of the loss sum
+// (y - x)^2 / T.
 //
 // k_stft_bwd: dL/dg_k = sum over windows (c_k/N) Re(X_k conj(E_k)), with X
 // the window's spectrum, E the spectrum of dL/dy over the window's outputs
@@ -48,6 +49,7 @@ struct StftArgs {
   float* lossp;        // [S][ntiles] or null
   float* gpart;        // [S][nblk][N/2 + 1] (backward)
   int S, T, H, ntiles, nblk, tile, rounds;
+  int logv;            // windows 2^logv hops apart do not overlap (forward)
   float invT;
 };
 
@@ -81,37 +83,46 @@ struct __attribute__((packed, aligned(4))) pair {
 
 // What a round costs is its VALU instructions, so everything a thread uses
 // again every round (window values, pass and bin-pair twiddles) is in
-// registers (within three waves per SIMD), windows inside the signal load without bounds tests, and a slot
-// adds its outputs to the tile itself.  Slots take runs of consecutive
-// windows (slot q the q-th R of them, one a round), so that a round's windows
-// lie R hops apart: with R H >= N they do not overlap and one barrier a round
-// orders the adds.  Shorter tiles take consecutive windows a round and add
-// them in ceil(N/H) phases.  (Gathering a round's outputs position by
-// position, 16 x 4 masked LDS reads a thread whatever the hop, took half of a
-// round's 1200 instructions: 114 us at 8 x 2^20 samples, N = 1024, H = 256;
-// 83 us so.)
+// registers (within three waves per SIMD), windows inside the signal load
+// without bounds tests, and a slot adds its outputs to the tile itself.
+//
+// The windows covering a sample are added by their residue w mod V, V the power
+// of two from N/H on, which differs for any two that overlap: an order that
+// depends on the windows' numbers alone, so a signal's y is the same bits
+// whatever the tile and the batch.  A tile's windows are taken residue by
+// residue, W at a time; those of one residue lie V hops apart, so one barrier
+// orders the adds of a round within a residue, and a round that runs into the
+// next residue adds one residue after the other.
+// (Gathering a round's outputs position by position, 16 x 4 masked LDS reads a
+// thread whatever the hop, took half of a round's 1200 instructions: 114 us at
+// 8 x 2^20 samples, N = 1024, H = 256; 85 us so.  Slots on consecutive runs of
+// windows instead, whose order depends on the tile, took 82.)
 template <int LOGN>
 __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
   constexpr int N = 1 << LOGN, M = N / 2, LOGM = LOGN - 1, P = M / 8, W = kThreads / P;
   constexpr int U = M / 2 / P + 1;  // bin pairs per thread
   // a window's P threads lie in one wave when P <= 64: its transforms and
-  // bins need only wave-level ordering; the gather reads every slot
+  // bins need only wave-level ordering; the adds to the tile cross slots
   constexpr bool WL = P <= 64;
   static_assert(W * M == 2048, "window slots must fill the FFT buffer");
-  extern __shared__ __align__(16) float acc[];  // [tile]
+  extern __shared__ __align__(16) float acc[];  // [tile, whole 64s], sample i at at(i)
+  // short windows: up to 16 slots of a wave add at once, N samples apart where H
+  // divides N; swapping a block's eights spreads them over the banks (8 x 2^20,
+  // N = 64, H = 16: 91 -> 77 us; at N = 256 and more it costs what it gives)
+  auto at = [](int i) { return LOGN <= 7 ? i ^ (((i >> 6) & 7) << 3) : i; };
   __shared__ c2 lbuf[2048];
   __shared__ float red[kThreads / 64];
   __shared__ float gain[M + 1];
-  const int tid = threadIdx.x, slot = tid / P, j = tid % P;
+  const int tid = threadIdx.x, j = tid % P;
+  const int slot = P >= 64 ? __builtin_amdgcn_readfirstlane(tid / P) : tid / P;
   const int s = blockIdx.y, tile = blockIdx.x, H = a.H;
   const int a0 = tile * a.tile, a1 = min(a.T, a0 + a.tile);
   const float* xs = a.x + (size_t)s * a.T;
   for (int i = tid; i <= M; i += kThreads) gain[i] = a.gains[i];
-  for (int i = tid; i < a.tile; i += kThreads) acc[i] = 0.0f;
+  for (int i = tid; i < ((a.tile + 63) & ~63); i += kThreads) acc[i] = 0.0f;
   // windows h = w*H with outputs [h, h+N) meeting [a0, a1)
   const int w_lo = a0 - N < 0 ? 0 : (a0 - N) / H + 1;
   const int w_hi = (a1 - 1) / H;
-  const int nw = w_hi - w_lo + 1;
   const SwzBuf buf(lbuf, slot * M);
   const int sj = buf.part(j);
   const HwRegTwiddle<LOGM> tw(j);
@@ -119,10 +130,18 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
   c2 wp[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) wp[u] = cis(-(float)(j + u * P) / (float)N);
-  const int rounds = (nw + W - 1) / W, V = (N + H - 1) / H;
-  const bool runs = rounds >= V;  // a round's windows do not overlap
-  const int phases = runs ? 1 : min(V, W), phase = runs ? 0 : slot % V;
-  auto window = [&](int r) { return w_lo + (runs ? slot * rounds + r : r * W + slot); };
+  // The tile's windows in that order, k = 0, 1, ...: before(q) have a residue
+  // below q; the first of residue q lies in block (of V) b0 or b0 + 1
+  const int logv = a.logv, V = 1 << logv, b0 = w_lo >> logv, rl = w_lo & (V - 1), rh = w_hi & (V - 1);
+  const int nw = w_hi - w_lo + 1, blocks = (w_hi >> logv) - b0 + 1;
+  auto before = [&](int q) { return q * blocks - min(q, rl) - max(q - rh - 1, 0); };
+  auto residue = [&](int k) {
+    int q = 0;
+    for (int b = V >> 1; b > 0; b >>= 1) q += before(q + b) <= k ? b : 0;
+    return q;
+  };
+  // (a slot past the last window has none)
+  auto window = [&](int k, int q) { return k < nw ? ((b0 + (q < rl) + k - before(q)) << logv) + q : w_hi + 1; };
   constexpr float invN = 1.0f / (float)N;
   // the window values this thread multiplies (samples 2n, 2n+1 of its first
   // pass inputs n), in registers for every round
@@ -132,12 +151,12 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
     const int n = in_pos<M, pass_radix(LOGM, 0)>(j, e);
     hw[e] = float2{a.win[2 * n], a.win[2 * n + 1]};
   }
-  // this thread's window samples of round r (element e of the first pass
+  // this thread's samples of window w (element e of the first pass
   // needs samples 2n and 2n+1 of the window, n = in_pos(j, e)); the next
   // round's are loaded while this one is transformed
   float px[16];
-  auto fetch = [&](int r) {
-    const int w = window(r), h = w * H, t00 = h - N + 1 + 2 * j;
+  auto fetch = [&](int w) {
+    const int h = w * H, t00 = h - N + 1 + 2 * j;
     if (__ballot(w > w_hi || h < N - 1) == 0) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -166,10 +185,10 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
       for (int e0 = 0; e0 < 8; e0 += 4) {
         float2 t[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) t[e] = *reinterpret_cast<const float2*>(acc + o + 2 * op[e0 + e]);
+        for (int e = 0; e < 4; ++e) t[e] = *reinterpret_cast<const float2*>(acc + at(o + 2 * op[e0 + e]));
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          *reinterpret_cast<float2*>(acc + o + 2 * op[e0 + e]) =
+          *reinterpret_cast<float2*>(acc + at(o + 2 * op[e0 + e])) =
               float2{t[e].x + v[e0 + e].x * invN, t[e].y + v[e0 + e].y * invN};
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -179,19 +198,30 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int i = o + 2 * op[e];
-      if (i >= 0 && i < a1 - a0) acc[i] += v[e].x * invN;
-      if (i + 1 >= 0 && i + 1 < a1 - a0) acc[i + 1] += v[e].y * invN;
+      if (i >= 0 && i < a1 - a0) acc[at(i)] += v[e].x * invN;
+      if (i + 1 >= 0 && i + 1 < a1 - a0) acc[at(i + 1)] += v[e].y * invN;
     }
   };
   __syncthreads();
-  fetch(0);
-  for (int r = 0; r < rounds; ++r) {
+  int q = residue(slot), w = window(slot, q);
+  int u = residue(0), end = before(u + 1);  // slot 0's residue, and its windows' end
+  fetch(w);
+  for (int k0 = 0; k0 < nw; k0 += W) {
     c2 v[8];
     int op[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = c2{px[2 * e] * hw[e].x, px[2 * e + 1] * hw[e].y};
     fft<LOGM, false, WL>(buf, j, v, op, tw);
-    if (r + 1 < rounds) fetch(r + 1);
+    const int wc = w, qc = q;  // this round's, for its adds
+    if (k0 + W < nw) {
+      if (k0 + 2 * W <= end) {
+        w += W << logv;
+      } else {
+        q = residue(k0 + W + slot);
+        w = window(k0 + W + slot, q);
+      }
+      fetch(w);
+    }
     fft_store<LOGM>(buf, j, v);
     lds_sync<WL>();
     // gains on the one-sided spectrum, then the Hermitian inverse
@@ -230,9 +260,16 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
     fft_load<LOGM>(buf, j, v);
     lds_sync<WL>();
     fft<LOGM, true, WL>(buf, j, v, op, tw);
-    for (int ph = 0; ph < phases; ++ph) {
-      if (phase == ph) add(window(r), v, op);
+    // a residue's adds at a time
+    const int kn = min(k0 + W, nw);
+    for (bool more = true; more;) {
+      if (qc == u) add(wc, v, op);
       lds_barrier();
+      more = end < kn;
+      if (end <= kn && end < nw) {
+        u = residue(end);
+        end = before(u + 1);
+      }
     }
   }
   float ls = 0.0f;
@@ -245,7 +282,7 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
     for (int q = 0; q < 8; ++q) {
       const int t = t8 + q * kThreads;
       if (t >= a1) break;
-      const float yv = acc[t - a0];
+      const float yv = acc[at(t - a0)];
       const float d = yv - xv[q];
       const size_t i = (size_t)s * a.T + t;
       if (a.y) a.y[i] = yv;
@@ -433,9 +470,10 @@ int launch_stft_fwd(const Launch& L, const dgen_hip_op& op) {
   a.H = (int)H;
   a.ntiles = (int)ntiles;
   a.tile = (int)tile;
+  while ((H << a.logv) < N) ++a.logv;
   a.invT = 1.0f / (float)T;
   hipLaunchKernelGGL(fwd_kernel(logn), dim3((unsigned)ntiles, (unsigned)S), dim3(kThreads),
-                     (unsigned)(tile * sizeof(float)), L.stream, a);
+                     (unsigned)((tile + 63) / 64 * 64 * sizeof(float)), L.stream, a);
   DGEN_LAUNCH_CHECK("k_stft_fwd");
   return 0;
 }

@@ -281,7 +281,8 @@ enum dgen_hip_kernel {
    * Forward: y, dL/dy = 2 (y - x)/T and per-tile loss partials sum
    * (y - x)^2 / T.  arg: [0]=x [1]=window [2]=gains [3]=y or -1 [4]=dy or -1
    * [5]=loss partials ([S][ceil(T/tile)]) or -1 [6]=S [7]=T [8]=N [9]=H
-   * [10]=tile (output samples per workgroup, 256..8192; 0: 8192) */
+   * [10]=tile (output samples per workgroup, 256..8192; 0: 8192; y and dy do
+   * not depend on it) */
   DGEN_HIP_K_STFT_FWD = 25,
 
   /* Gain gradient partials: row (s, b) sums (c_k/N) Re(X_k conj(E_k)) over

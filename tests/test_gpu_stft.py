@@ -152,11 +152,10 @@ def test_full_configuration_matches_oracle(gpu):
                                      (2, 20000, 2048, 512), (1, 9000, 2048, 2048)])
 @pytest.mark.parametrize("tile,rounds", [(256, 1), (257, 1), (512, 2), (1280, 3), (1281, 3), (8192, 8)])
 def test_tiles_and_rounds_agree_with_the_oracle(gpu, S, T, N, H, tile, rounds):
-    """Output tiles and gradient runs of any length: windows added in phases
-    (tiles shorter than the windows of a round span) or a run per slot, odd
-    hops and tiles, hops of 1 and of N.  A position's sum of up to N/H windows
-    is only reordered, so y keeps test_forward_matches_oracle's bar and the
-    loss and gradient the fp32 oracle's distance from fp64."""
+    """Output tiles and gradient runs of any length, odd hops and tiles, hops
+    of 1 and of N.  A position's sum of up to N/H windows is only reordered, so
+    y keeps test_forward_matches_oracle's bar and the loss and gradient the
+    fp32 oracle's distance from fp64."""
     cfg = StftConfig(S=S, T=T, N=N, H=H)
     x, g = cfg.inputs(), random_gains(cfg.bins, N + T)
     print(f"case S={S} T={T} N={N} H={H} tile={tile} rounds={rounds}", flush=True)
@@ -180,3 +179,32 @@ def test_tiles_and_rounds_agree_with_the_oracle(gpu, S, T, N, H, tile, rounds):
     assert abs(loss - l64) <= 8.0 * abs(l32 - l64) + 2e-6 * abs(l64)
     n = np.linalg.norm
     assert n(dg - g64) <= 8.0 * n(g32 - g64) + 2e-6 * n(g64)
+
+
+@pytest.mark.parametrize("T,N,H", [(9001, 64, 16), (3000, 64, 1), (9001, 128, 33), (20003, 256, 64), (30001, 512, 128),
+                                   (9000, 1024, 100), (30001, 1024, 256), (30001, 2048, 512), (20003, 2048, 700)])
+def test_audio_does_not_depend_on_the_tile_or_the_batch(gpu, T, N, H):
+    """A sample's windows are added in an order of their own, so a signal's y
+    and dL/dy are the same bits for any tile length, alone or in a batch (whose
+    size picks the builder's tile)."""
+    cfg = StftConfig(S=9, T=T, N=N, H=H)
+    x, g = cfg.inputs(), random_gains(cfg.bins, N + T)
+
+    def forward(xs, tile):
+        S = len(xs)
+        p = Program(max_frames=T)
+        c = {n: p.alloc(n, k) for n, k in (("x", S * T), ("window", N), ("gains", cfg.bins), ("y", S * T),
+                                           ("dy", S * T))}
+        p.add(R.K_STFT_FWD, [c["x"], c["window"], c["gains"], c["y"], c["dy"], -1, S, T, N, H, tile])
+        with HIPLazyRuntime(p) as rt:
+            for n, a in (("x", xs), ("window", cfg.window()), ("gains", g)):
+                rt.write(n, a)
+            rt.runNoCopy()
+            return rt.read("y").reshape(S, T), rt.read("dy").reshape(S, T)
+
+    want = forward(x, 8192)
+    for tile in (256, 512, 1000, 1024, 1281, 2048, 4096):
+        print(f"case T={T} N={N} H={H} tile={tile}", flush=True)
+        for a, b in zip(forward(x[:2], tile), want):
+            np.testing.assert_array_equal(a, b[:2])
+    np.testing.assert_array_equal(render(StftConfig(S=1, T=T, N=N, H=H), x[:1], g), want[0][:1])
