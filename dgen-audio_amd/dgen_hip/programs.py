@@ -15,11 +15,6 @@ from .workloads import (BiquadConfig, HarmonicConfig, MembraneConfig, OscBankCon
                         SweptPhasorConfig)
 
 
-class DefaultChunk(int):
-    """A scan's chunk length as the builders choose it, so that they may
-    shorten it (`_scan_chunk`); a plain int is a caller's and is kept."""
-
-
 SEG = 64          # frames per synth segment (checkpoint spacing)
 SLOTS = 4         # control rows a segment may touch
 ROW_ENTRIES = 16  # (segment, slot) entries per control row (kRowEntries)
@@ -32,8 +27,8 @@ GEMM_TILE_M = 128  # output rows per GEMM workgroup tile (k_gemm.hip BM)
 GEMM_SMALL_TILES = 128  # 128 x 128 tiles up to which a split-bf16 GEMM splits its own operands (k_gemm.hip kSmTiles)
 SPLITK_ROWS_HEADS = 256  # the heads' weight gradient has one 128-wide column tile: split finer to fill the chip
 MSS_TILE = 4096     # output samples per spectral-loss workgroup
-BQ_CHUNK = DefaultChunk(512)   # frames per biquad scan chunk (512 measured fastest of 128..1024)
-SVF_CHUNK = DefaultChunk(256)  # frames per SVF scan chunk
+BQ_CHUNK = 512      # frames per biquad scan chunk (512 measured fastest of 128..1024)
+SVF_CHUNK = 256     # frames per SVF scan chunk
 SCAN_WAVES = 2048   # waves (64 lanes x one chunk) a filter scan's passes should have: two per SIMD
 STFT_TILE = 8192    # largest output tile of an STFT forward workgroup
 STFT_GROUPS = 512   # workgroups an STFT pass is split into if need be (two per CU)
@@ -456,19 +451,21 @@ class HarmonicSession:
 
 
 # ------------------------------------------------------------------ config 4
-def _scan_chunk(B: int, T: int, chunk: int) -> int:
-    """Frames per chunk of a filter bank's scans: `chunk`, a default one halved
-    (to no less than 32, in whole thirty-twos) while the lanes and chunks make
-    fewer than SCAN_WAVES waves.  A pass lasts as long as one chunk's frames in sequence
-    (~0.25 us each), so few lanes or a short signal want shorter chunks; with
+def _scan_chunk(B: int, T: int, chunk: int | None, default: int) -> int:
+    """Frames per chunk of a filter bank's scans: the caller's `chunk`, or, if
+    it names none, `default` halved (to no less than 32, in whole thirty-twos)
+    while the lanes and chunks make fewer than SCAN_WAVES waves.  A pass lasts
+    as long as one chunk's frames in sequence (~0.25 us each), so few lanes or a short signal want shorter chunks; with
     the chip full, shorter ones only add chunk maps to the carry.  Steps
     measured: biquad 12 lanes x 8192 frames 488 us at 512, 134 at 32, 137 at
     16; linear SVF 70 x 30001 368 us at 256, 216 at 64, 197 at 32, 236 at 16;
     saturating SVF 256 x 65536 814 us at 256, 755 at 128, 765 at 64; biquad 256
     x 2^18 605 us at 512 (kept), 624 at 256, 678 at 128."""
-    L, groups = int(chunk), (B + 63) // 64
-    if not isinstance(chunk, DefaultChunk):
-        return L
+    if chunk is not None:
+        if int(chunk) <= 0:
+            raise ValueError("chunk length must be positive")
+        return int(chunk)
+    L, groups = default, (B + 63) // 64
     while L % 64 == 0 and groups * ((T + L - 1) // L) < SCAN_WAVES:
         L //= 2
     return L
@@ -479,7 +476,7 @@ def _colsum_ws(rows: int, cols: int) -> int:
 
 
 def biquad_program(cfg: BiquadConfig, train: bool = True, optimizer: bool = True, modulated: bool = True,
-                   chunk: int = BQ_CHUNK, fuse_adjoint: bool = True) -> Program:
+                   chunk: int | None = None, fuse_adjoint: bool = True) -> Program:
     """Tensor biquad bank: x -> RBJ low-pass with cutoff base[k]*mod[n] and Q[k].
 
     ``train=False`` builds the forward render only (used for the fixed target
@@ -490,10 +487,8 @@ def biquad_program(cfg: BiquadConfig, train: bool = True, optimizer: bool = True
     ``fuse_adjoint`` the forward replay also forms the adjoint's chunk
     summaries; without it a separate reverse pass over y and the target
     does."""
-    B, T, L = cfg.B, cfg.T, int(chunk)
-    if L <= 0:
-        raise ValueError("chunk length must be positive")
-    L = _scan_chunk(B, T, chunk)
+    B, T = cfg.B, cfg.T
+    L = _scan_chunk(B, T, chunk, BQ_CHUNK)
     C = (T + L - 1) // L
     f4 = 4.0
     p = Program(max_frames=T)
@@ -586,7 +581,7 @@ class BiquadSession:
     forward-only program with the fixed (tgt_fc, tgt_Q) coefficients, then
     every ``step()`` is forward + loss + BPTT (+ Adam) with all data in HBM."""
 
-    def __init__(self, cfg: BiquadConfig, device: int = 0, optimizer: bool = True, chunk: int = BQ_CHUNK,
+    def __init__(self, cfg: BiquadConfig, device: int = 0, optimizer: bool = True, chunk: int | None = None,
                  target=None, fuse_adjoint: bool = True):
         self.cfg = cfg
         self.x = cfg.inputs()
@@ -602,7 +597,7 @@ class BiquadSession:
         self.rt.write("params", self.params0)
         self.rt.write("target", self.target)
 
-    def render(self, params, device: int = 0, modulated: bool = True, chunk: int = BQ_CHUNK) -> np.ndarray:
+    def render(self, params, device: int = 0, modulated: bool = True, chunk: int | None = None) -> np.ndarray:
         prog = biquad_program(self.cfg, train=False, modulated=modulated, chunk=chunk)
         with R.HIPLazyRuntime(prog, device) as rt:
             rt.write("x", self.x)
@@ -624,7 +619,7 @@ class BiquadSession:
 
 # ------------------------------------------------------ ZDF SVF bank (BPTT)
 def svf_program(cfg: SvfConfig, train: bool = True, optimizer: bool = True, saturating: bool | None = None,
-                chunk: int = SVF_CHUNK, xbar: bool = False, fuse_adjoint: bool = True) -> Program:
+                chunk: int | None = None, xbar: bool = False, fuse_adjoint: bool = True) -> Program:
     """ZDF SVF low-pass bank: x -> y with cutoff clip(base[k]*mod[n] + env[n])
     and res[k] (and, saturating, kSat[k]).
 
@@ -638,11 +633,9 @@ def svf_program(cfg: SvfConfig, train: bool = True, optimizer: bool = True, satu
     adjoint's chunk summaries, else a separate reverse pass over y and the
     target does."""
     sat = cfg.saturating if saturating is None else bool(saturating)
-    B, T, L = cfg.B, cfg.T, int(chunk)
-    if L <= 0:
-        raise ValueError("chunk length must be positive")
+    B, T = cfg.B, cfg.T
     P = 3 if sat else 2
-    L = _scan_chunk(B, T, chunk)
+    L = _scan_chunk(B, T, chunk, SVF_CHUNK)
     C = (T + L - 1) // L
     f4 = 4.0
     n = float(T * B)
@@ -747,7 +740,7 @@ class SvfSession:
     forward-only program with (tgt_fc, tgt_res), then every ``step()`` is
     forward + loss + BPTT (+ Adam) with all data in HBM."""
 
-    def __init__(self, cfg: SvfConfig, device: int = 0, optimizer: bool = True, chunk: int = SVF_CHUNK,
+    def __init__(self, cfg: SvfConfig, device: int = 0, optimizer: bool = True, chunk: int | None = None,
                  target=None, xbar: bool = False, fuse_adjoint: bool = True):
         self.cfg = cfg
         self.x = cfg.inputs()
@@ -764,7 +757,7 @@ class SvfSession:
                         ("target", self.target)):
             self.rt.write(name, a)
 
-    def render(self, params, device: int = 0, saturating: bool = False, chunk: int = SVF_CHUNK) -> np.ndarray:
+    def render(self, params, device: int = 0, saturating: bool = False, chunk: int | None = None) -> np.ndarray:
         prog = svf_program(self.cfg, train=False, saturating=saturating, chunk=chunk)
         with R.HIPLazyRuntime(prog, device) as rt:
             for name, a in (("x", self.x), ("mod", self.mod), ("env", self.env), ("params", params)):

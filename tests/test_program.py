@@ -6,9 +6,10 @@ import pytest
 from dgen_hip import HarmonicConfig
 from dgen_hip import runtime as R
 from dgen_hip.program import ALIGN, Program
-from dgen_hip.programs import harmonic_program, oscbank_program
+from dgen_hip.programs import (BQ_CHUNK, SVF_CHUNK, biquad_program, harmonic_program, oscbank_program,
+                               svf_program)
 from dgen_hip.roofline import roof_seconds, step_roof_ms
-from dgen_hip.workloads import OscBankConfig, SplitMix64
+from dgen_hip.workloads import BiquadConfig, OscBankConfig, SplitMix64, SvfConfig
 
 
 def test_cells_are_aligned_and_disjoint():
@@ -106,3 +107,17 @@ def test_oscbank_inputs_follow_config():
     freqs, amps = OscBankConfig().inputs()
     np.testing.assert_array_equal(freqs, (np.arange(1, 17) * 220.0).astype(np.float32))
     assert abs(float(amps.sum()) - 1.0) < 1e-6
+
+
+@pytest.mark.parametrize("chunk", [1, 96, BQ_CHUNK, SVF_CHUNK, np.int64(512)])
+def test_a_named_scan_chunk_is_kept(chunk):
+    """The builders shorten only their own chunk length; one that the caller
+    names is kept, the module's constants included."""
+    for prog in (biquad_program(BiquadConfig(B=12, T=8192), chunk=chunk),
+                 svf_program(SvfConfig(B=12, T=8192), chunk=chunk)):
+        assert prog.meta["chunk"] == chunk and prog.meta["chunks"] == -(-8192 // int(chunk))
+    for bad in (0, -32):
+        with pytest.raises(ValueError, match="positive"):
+            biquad_program(BiquadConfig(B=12, T=8192), chunk=bad)
+        with pytest.raises(ValueError, match="positive"):
+            svf_program(SvfConfig(B=12, T=8192), chunk=bad)
