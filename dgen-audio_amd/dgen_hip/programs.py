@@ -29,7 +29,7 @@ SPLITK_ROWS_HEADS = 256  # the heads' weight gradient has one 128-wide column ti
 MSS_TILE = 4096     # output samples per spectral-loss workgroup
 BQ_CHUNK = 512      # frames per biquad scan chunk (512 measured fastest of 128..1024)
 SVF_CHUNK = 256     # frames per SVF scan chunk
-SCAN_WAVES = 2048   # waves (64 lanes x one chunk) a filter scan's passes should have: two per SIMD
+SCAN_CHUNKS = 512   # chunks a filter scan should have: two waves per SIMD at 256 lanes
 STFT_TILE = 8192    # largest output tile of an STFT forward workgroup
 STFT_GROUPS = 512   # workgroups an STFT pass is split into if need be (two per CU)
 MEM_STEPS = 16      # membrane frames per time-blocked launch
@@ -451,22 +451,28 @@ class HarmonicSession:
 
 
 # ------------------------------------------------------------------ config 4
-def _scan_chunk(B: int, T: int, chunk: int | None, default: int) -> int:
+def _scan_chunk(T: int, chunk: int | None, default: int) -> int:
     """Frames per chunk of a filter bank's scans: the caller's `chunk`, or, if
     it names none, `default` halved (to no less than 32, in whole thirty-twos)
-    while the lanes and chunks make fewer than SCAN_WAVES waves.  A pass lasts
-    as long as one chunk's frames in sequence (~0.25 us each), so few lanes or a short signal want shorter chunks; with
-    the chip full, shorter ones only add chunk maps to the carry.  Steps
-    measured: biquad 12 lanes x 8192 frames 488 us at 512, 134 at 32, 137 at
-    16; linear SVF 70 x 30001 368 us at 256, 216 at 64, 197 at 32, 236 at 16;
-    saturating SVF 256 x 65536 814 us at 256, 755 at 128, 765 at 64; biquad 256
-    x 2^18 605 us at 512 (kept), 624 at 256, 678 at 128."""
+    while a signal has fewer than SCAN_CHUNKS chunks.  The number of lanes has
+    no say: a chunk's length sets where a lane's fp32 states are rounded, and a
+    lane gives the same bits in every bank.
+
+    A pass lasts as long as one chunk's frames in sequence (~0.25 us each), so
+    a short signal wants short chunks; with the chip full, shorter ones only add
+    chunk maps to the carry.  Training steps measured, us at 32 / 64 / 128 / 256
+    / 512 frames: biquad 256 lanes x 2^13 64 / 77 / 113 / 191 / 350, x 2^16 253
+    / 183 / 168 / 212 / 367, x 2^18 1011 / 708 / 590 / 538 / 505; 64 lanes x
+    2^16 144 / 117 / 131 / 190 / 337, x 2^18 513 / 306 / 255 / 258 / 374; 2048
+    lanes x 2^13 178 / 151 / 152 / 203 / 362; linear SVF (to 256) 256 lanes x
+    2^16 340 / 267 / 258 / 311, 4 lanes x 2^16 161 / 230 / 273 / 353; the
+    saturating one changes by a few percent."""
     if chunk is not None:
         if int(chunk) <= 0:
             raise ValueError("chunk length must be positive")
         return int(chunk)
-    L, groups = default, (B + 63) // 64
-    while L % 64 == 0 and groups * ((T + L - 1) // L) < SCAN_WAVES:
+    L = default
+    while L % 64 == 0 and (T + L - 1) // L < SCAN_CHUNKS:
         L //= 2
     return L
 
@@ -488,7 +494,7 @@ def biquad_program(cfg: BiquadConfig, train: bool = True, optimizer: bool = True
     summaries; without it a separate reverse pass over y and the target
     does."""
     B, T = cfg.B, cfg.T
-    L = _scan_chunk(B, T, chunk, BQ_CHUNK)
+    L = _scan_chunk(T, chunk, BQ_CHUNK)
     C = (T + L - 1) // L
     f4 = 4.0
     p = Program(max_frames=T)
@@ -635,7 +641,7 @@ def svf_program(cfg: SvfConfig, train: bool = True, optimizer: bool = True, satu
     sat = cfg.saturating if saturating is None else bool(saturating)
     B, T = cfg.B, cfg.T
     P = 3 if sat else 2
-    L = _scan_chunk(B, T, chunk, SVF_CHUNK)
+    L = _scan_chunk(T, chunk, SVF_CHUNK)
     C = (T + L - 1) // L
     f4 = 4.0
     n = float(T * B)

@@ -185,3 +185,22 @@ def test_chunk_limit_is_an_error(gpu):
     cfg = BiquadConfig(B=1, T=70000)
     with pytest.raises(HIPError, match="chunks"):
         HIPLazyRuntime(biquad_program(cfg, train=False, chunk=1), 0)
+
+
+def test_a_lane_does_not_depend_on_its_bank(gpu):
+    """The first lanes of a bank of 300 give the audio and the gradient of a
+    bank of their own, bit for bit, at the builders' chunk length."""
+    T, few = 40000, 5
+    wide, cfg = BiquadConfig(B=300, T=T), BiquadConfig(B=few, T=T)
+    x, mod = wide.inputs(), wide.modulation()
+    tgt = np.random.default_rng(1).uniform(-1, 1, x.shape).astype(np.float32)
+    prm = np.stack(lane_params(300, 2))
+    got = []
+    for c in (wide, cfg):
+        with HIPLazyRuntime(biquad_program(c, optimizer=False)) as rt:
+            for name, a in (("x", x[:, :c.B]), ("target", tgt[:, :c.B]), ("mod", mod), ("params", prm[:, :c.B])):
+                rt.write(name, a)
+            rt.runNoCopy()
+            got.append((rt.read("y").reshape(T, -1)[:, :few], rt.read("grads").reshape(2, -1)[:, :few]))
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)

@@ -231,3 +231,23 @@ def test_saturating_spans_equal_the_frame_loop(B, T, chunk, signal):
         bits = [np.where(np.isnan(v), 0, v.view(np.uint32)) for v in (a, b)]  # a NaN's sign is not defined
         np.testing.assert_array_equal(np.isnan(a), np.isnan(b))
         np.testing.assert_array_equal(*bits)
+
+
+@pytest.mark.parametrize("saturating", [False, True])
+def test_a_lane_does_not_depend_on_its_bank(gpu, saturating):
+    """The first lanes of a bank of 300 give the audio and the gradient of a
+    bank of their own, bit for bit, at the builders' chunk length."""
+    T, few = 40000, 5
+    wide, cfg = (SvfConfig(B=B, T=T, saturating=saturating) for B in (300, few))
+    x, tgt = (np.random.default_rng(s).uniform(-1, 1, (T, 300)).astype(np.float32) for s in (1, 2))
+    prm = wide.params().reshape(-1, 300)
+    got = []
+    for c in (wide, cfg):
+        with HIPLazyRuntime(svf_program(c, optimizer=False)) as rt:
+            for name, a in (("x", x[:, :c.B]), ("target", tgt[:, :c.B]), ("mod", wide.modulation()),
+                            ("env", wide.envelope()), ("params", prm[:, :c.B])):
+                rt.write(name, a)
+            rt.runNoCopy()
+            got.append((rt.read("y").reshape(T, -1)[:, :few], rt.read("grads").reshape(len(prm), -1)[:, :few]))
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)

@@ -121,3 +121,13 @@ def test_a_named_scan_chunk_is_kept(chunk):
             biquad_program(BiquadConfig(B=12, T=8192), chunk=bad)
         with pytest.raises(ValueError, match="positive"):
             svf_program(SvfConfig(B=12, T=8192), chunk=bad)
+
+
+@pytest.mark.parametrize("T", [1, 31, 2048, 8192, 30001, 40000, 1 << 18])
+def test_scan_chunks_do_not_depend_on_the_bank(T):
+    """A lane's samples are rounded to fp32 at its chunks' edges, so the
+    default chunk length follows the signal's length alone."""
+    for build, cfg in ((biquad_program, BiquadConfig), (svf_program, SvfConfig)):
+        chunks = {build(cfg(B=B, T=T)).meta["chunk"] for B in (1, 5, 64, 65, 256, 1000)}
+        assert len(chunks) == 1
+        assert chunks.pop() % 32 == 0
