@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <cstdio>
+#include <initializer_list>
 
 #include "../../include/dgen_hip.h"
 
@@ -47,6 +48,26 @@ int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 // Cell-range check: [off, off+n) inside the arena and off >= 0.
 int check_cell(const Launch& L, int64_t off, uint64_t n, const char* what);
 inline float* cell(const Launch& L, int64_t off) { return L.arena + off; }
+
+// Cells [off, off+n) of an op; none where off is negative.
+struct CellRange {
+  int64_t off, n;
+};
+// True if the ranges an op writes share no cell with one another or with any
+// it reads (which may share cells among themselves).  Schedules that write a
+// cell before its last read, or more than once, are for such ops only.
+inline bool written_apart(std::initializer_list<CellRange> written, std::initializer_list<CellRange> read) {
+  auto apart = [](const CellRange& a, const CellRange& b) {
+    return a.off < 0 || b.off < 0 || a.off + a.n <= b.off || b.off + b.n <= a.off;
+  };
+  for (auto w = written.begin(); w != written.end(); ++w) {
+    for (auto v = written.begin(); v != w; ++v)
+      if (!apart(*w, *v)) return false;
+    for (const CellRange& r : read)
+      if (!apart(*w, r)) return false;
+  }
+  return true;
+}
 
 #define DGEN_CHECK_CELL(L, off, n, what)                      \
   do {                                                        \

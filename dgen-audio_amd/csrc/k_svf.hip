@@ -969,9 +969,15 @@ int launch_svf_seq(const Launch& L, const dgen_hip_op& op) {
   float* lp = lossp >= 0 ? cell(L, lossp) : nullptr;
   const int64_t groups = (s.B + 63) / 64;
   const int64_t per = std::max<int64_t>((kSpecSpan + s.L - 1) / s.L, groups * s.C / (4 * L.cu_count));
+  // the spans read their inputs several times and keep states between passes,
+  // so nothing they write may share cells with anything else (the loop reads a
+  // frame before it writes it, and works in place)
+  const int64_t n = s.B * s.T;
+  const bool apart = spec && written_apart({{y, n}, {cl, 2 * n}, {lossp, s.C * s.B}, {op.arg[14], 6 * s.C * s.B}},
+                                           {{x, n}, {prm, 3 * s.B}, {tgt, n}, {tape, n}});
   // the spans keep the training step's outputs (all or y alone), take whole
   // prefetch groups to a loss chunk and address a span's rows in 31 bits
-  if (spec && s.C > 1 && !san && (tgt >= 0) == (cl >= 0) && s.L % kSpecG == 0 && per * s.L * s.B < (1ll << 28)) {
+  if (apart && s.C > 1 && !san && (tgt >= 0) == (cl >= 0) && s.L % kSpecG == 0 && per * s.L * s.B < (1ll << 28)) {
     // spans of whole loss chunks, at least kSpecSpan frames, longer where the
     // lanes alone give every SIMD a wave: a pass then still fills the chip
     // once and each one extends what a span has seen by more

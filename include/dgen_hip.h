@@ -397,7 +397,8 @@ enum dgen_hip_kernel {
    *      [14]=span states (6*C*B floats, C = ceil(T/L)) when [15]=1: spans of
    *      frames run side by side from speculated states, repeated until each
    *      starts bit for bit where the one before ends (the same results; needs
-   *      the tape and no state cell)
+   *      the tape and no state cell; where y, cells, partials or span states
+   *      share cells with one another or an input, frame by frame as without)
    * With a target, cells and a tape, B a multiple of 64 and T and L of 32,
    * the loop runs on 32-frame LDS tiles (the same results). */
   DGEN_HIP_K_SVF_SEQ = 35,

@@ -10,6 +10,7 @@ import pytest
 import oracle as O
 from dgen_hip import SvfConfig
 from dgen_hip import runtime as R
+from dgen_hip.program import Program
 from dgen_hip.programs import SvfSession, stream_svf_program, svf_program
 from dgen_hip.runtime import HIPLazyRuntime
 
@@ -249,5 +250,35 @@ def test_a_lane_does_not_depend_on_its_bank(gpu, saturating):
                 rt.write(name, a)
             rt.runNoCopy()
             got.append((rt.read("y").reshape(T, -1)[:, :few], rt.read("grads").reshape(len(prm), -1)[:, :few]))
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("shared", ["y is x", "y is the target", "y is the tape", "cells end in x", "spans in y"])
+def test_spans_asked_for_in_place_run_frame_by_frame(gpu, shared):
+    """An op that asks for spans and writes over its inputs (or keeps the span
+    states in an output) leaves what the frame loop leaves."""
+    B, T, L = 5, 4000, 96
+    cfg, n = SvfConfig(B=B, T=T, saturating=True), B * T
+    C = -(-T // L)
+    x, tgt = (np.random.default_rng(s).uniform(-1, 1, n).astype(np.float32) for s in (1, 2))
+    got = []
+    for spans in (0, 1):
+        p = Program(max_frames=T)
+        c = {k: p.alloc(k, m) for k, m in (("cells", 2 * n), ("x", n), ("target", n), ("y", n), ("tape", n),
+                                           ("mod", T), ("env", T), ("params", 3 * B), ("loss", C * B),
+                                           ("states", 6 * C * B))}
+        y = {"y is x": c["x"], "y is the target": c["target"], "y is the tape": c["tape"]}.get(shared, c["y"])
+        cells = c["x"] - n if shared == "cells end in x" else c["cells"]
+        states = c["y"] if shared == "spans in y" else c["states"]
+        p.add(R.K_SVF_SEQ, [c["x"], c["mod"], c["env"], c["params"], -1, y, cells, c["target"], c["loss"], B, T, L, 0,
+                            c["tape"], states, spans], [cfg.sr])
+        print(f"case {shared}, spans {spans}", flush=True)
+        with HIPLazyRuntime(p) as rt:
+            for name, a in (("x", x), ("target", tgt), ("mod", cfg.modulation()), ("env", cfg.envelope()),
+                            ("params", cfg.params())):
+                rt.write(name, a)
+            rt.runNoCopy()
+            got.append([rt.read(k) for k in ("x", "target", "y", "tape", "loss")])
     for a, b in zip(*got):
         np.testing.assert_array_equal(a, b)
