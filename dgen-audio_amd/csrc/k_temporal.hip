@@ -458,9 +458,13 @@ int launch_swept_phasor(const Launch& L, const dgen_hip_op& op) {
   }
   if (L.dry) return 0;
   // the passes need one whole quad and their blocks in the grid's second
-  // dimension; other lengths, and ops without scratch, take the one-pass loop
+  // dimension, and read slopes, times, resets and scratch after their first
+  // writes; other lengths, ops that write over their inputs and ops without
+  // scratch take the one-pass loop
   const int64_t groups = (E + 63) / 64, yblk = (T / kSpSeg + 3) / 4, yseg = (sp_segments((int)T) + 3) / 4;
-  if (scratch && T >= 4 && yblk <= 65535 && yseg <= 65535) {
+  const bool apart = scratch && written_apart({{ph, E * T}, {gu, E * T}, {lp, E}, {op.arg[9], E * T}},
+                                              {{sl, E}, {tm, T}, {rs, T}});
+  if (apart && T >= 4 && yblk <= 65535 && yseg <= 65535) {
     const float sr = host_rate(L, op.farg[0]), base = op.farg[1];
     const float* rp = rs >= 0 ? cell(L, rs) : nullptr;
     float4* tape = reinterpret_cast<float4*>(cell(L, op.arg[9]));

@@ -357,7 +357,8 @@ enum dgen_hip_kernel {
    *      ([T][E]) or -1 [4]=upstream ([T][E]) [5]=loss partials ([E]) [6]=E
    *      [7]=T [8]=smooth (0/1) [9]=scratch ([T][E], 16-byte aligned) when [10]=1
    *      (the increments are formed ahead of the phase chain; its contents are
-   *      not defined afterwards)
+   *      not defined afterwards; where phase, upstream, partials or scratch
+   *      share cells with one another or an input, frame by frame as without)
    * farg: [0]=sample rate [1]=base frequency [2]=target */
   DGEN_HIP_K_SWEPT_PHASOR = 32,
 

@@ -71,7 +71,7 @@ def test_scan_matches_oracle(gpu, E, T):
 def test_swept_phasor_passes_equal_the_one_pass_loop(E, T, form):
     """With a scratch cell the increments, the phase chain and the loss run as
     separate passes: phase and upstream gradient are the one-pass loop's bit
-    for bit over every edge of the blocks of 32 and segments of 64 frames,
+    for bit over every edge of the 64-frame intervals and segments,
     with resets, negative increments and non-finite ones; the loss, fp64 sums
     in another order rounded to fp32 at the end, to one ulp (1.2e-7)."""
     rng = np.random.default_rng(E * 7 + T)
@@ -96,6 +96,38 @@ def test_swept_phasor_passes_equal_the_one_pass_loop(E, T, form):
     for a, b in zip(got[0][:2], got[1][:2]):
         np.testing.assert_array_equal(a, b)
     np.testing.assert_allclose(got[1][2], got[0][2], rtol=1.2e-7)
+
+
+@pytest.mark.parametrize("shared", ["upstream over the slopes", "loss over the slopes", "phase is upstream",
+                                    "scratch is upstream", "scratch is phase"])
+def test_swept_phasor_in_place_runs_in_one_pass(gpu, shared):
+    """An op with a scratch cell that writes over its inputs, or whose scratch
+    is one of its outputs, leaves what the one-pass loop leaves."""
+    E, T = 40, 1027
+    rng = np.random.default_rng(3)
+    slope, time = rng.uniform(100, 3e4, E), np.arange(T) / 44100.0
+    got = []
+    for scratch in (0, 1):
+        p = Program(max_frames=T)
+        c = {n: p.alloc(n, k) for n, k in (("time", T), ("reset", T), ("phase", T * E), ("g", T * E), ("loss", E),
+                                           ("scratch", T * E), ("slope", E))}
+        sl = {"upstream over the slopes": c["g"]}.get(shared, c["slope"])
+        lp = sl if shared == "loss over the slopes" else c["loss"]
+        ph = c["g"] if shared == "phase is upstream" else c["phase"]
+        sc = {"scratch is upstream": c["g"], "scratch is phase": c["phase"]}.get(shared, c["scratch"])
+        p.add(R.K_SWEPT_PHASOR, [sl, c["time"], c["reset"], ph, c["g"], lp, E, T, 1, sc, scratch],
+              [44100.0, 80.0, 0.08])
+        print(f"case {shared}, scratch {scratch}", flush=True)
+        with R.HIPLazyRuntime(p) as rt:
+            for n, a in (("slope", slope), ("time", time)):
+                rt.write(n, a)
+            if sl == c["g"]:
+                rt.write("g", np.concatenate([slope, np.zeros(T * E - E)]))
+            rt.runNoCopy()
+            got.append([rt.read(n) for n in ("phase", "g", "loss", "slope")])
+    assert np.abs(got[0][1]).max() > 0
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
 
 
 @pytest.mark.parametrize("reset_from", [-1, 40000])
