@@ -750,6 +750,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 // 38.9, 64 70.9 / 43.2, 128 74.1 / 67.0, 256 82.0 / 89.2: up to kSmTiles.
 constexpr int kSmDepth = 4;
 constexpr int64_t kSmTiles = 128;
+// Its lanes address operands by 32-bit byte offsets, and values of a plane
+// ([K8][N]) by int indices.
+constexpr bool fits_x6s(int64_t tiles, int64_t bytes_a, int64_t bytes_b, bool planes, int64_t K8, int64_t N) {
+  return tiles <= kSmTiles && bytes_a < (1ll << 31) && (planes ? K8 * N < (1ll << 31) : bytes_b < (1ll << 31));
+}
+static_assert(fits_x6s(128, 4, 0, true, 1 << 17, (1 << 14) - 1) && !fits_x6s(128, 4, 0, true, 1 << 17, 1 << 14),
+              "a plane of 2^31 values is out of an int index's reach");
+static_assert(fits_x6s(128, 4, 4, false, 1 << 17, 1 << 14) && !fits_x6s(129, 4, 4, false, 1, 1) &&
+                  !fits_x6s(1, 1ll << 31, 4, false, 1, 1) && !fits_x6s(1, 4, 1ll << 31, false, 1, 1),
+              "tiles and byte offsets");
 template <bool A_KMAJ, bool B_NK, bool BPL, bool VEC>
 __global__ __launch_bounds__(128) void k_gemm_x6s(const float* __restrict__ A, const float* __restrict__ B,
                                                   float* __restrict__ C, int M, int N, int K, int lda, int ldb,
@@ -1183,7 +1193,7 @@ int launch_gemm(const Launch& L, const dgen_hip_op& op) {
 #define DGEN_X6L(AK_, BT_)                                                                                          \
   launch_x6<AK_, BT_>(va, vb, full6, g, L.stream, pa, pb, pc, M, N, K, lda, ldb, ldc, e, pbias, paux, ldaux, kchunk, \
                       pws, pcs, pcw, ncw, pbpl, (int)K8)
-    if ((int64_t)g.x * g.y * g.z <= kSmTiles && ext_a < (1ll << 31) && (pbpl || ext_b < (1ll << 31))) {
+    if (fits_x6s((int64_t)g.x * g.y * g.z, ext_a, ext_b, pbpl != nullptr, K8, N)) {
       const dim3 gs((unsigned)((N + 31) / 32), g.y, g.z);
       auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, gs, dim3(128), 0, L.stream, pa, pb, pc, (int)M, (int)N, (int)K, (int)lda, (int)ldb,
