@@ -1193,7 +1193,14 @@ int launch_gemm(const Launch& L, const dgen_hip_op& op) {
 #define DGEN_X6L(AK_, BT_)                                                                                          \
   launch_x6<AK_, BT_>(va, vb, full6, g, L.stream, pa, pb, pc, M, N, K, lda, ldb, ldc, e, pbias, paux, ldaux, kchunk, \
                       pws, pcs, pcw, ncw, pbpl, (int)K8)
-    if (fits_x6s((int64_t)g.x * g.y * g.z, ext_a, ext_b, pbpl != nullptr, K8, N)) {
+    // (one 128 x 128 tile may write over its operands: a single workgroup reads
+    // them whole before it stores, where k_gemm_x6s has several)
+    const std::initializer_list<CellRange> operands = {
+        {A, alay == 0 ? (M - 1) * lda + K : (K - 1) * lda + M},
+        pbpl ? CellRange{planes, 3 * K8 * N * 4} : CellRange{Bc, blay == 0 ? (K - 1) * ldb + N : (N - 1) * ldb + K}};
+    const bool apart = pws ? written_apart({{ws, splits * M * N}}, operands)
+                           : written_apart({{Cc, (M - 1) * ldc + N}}, operands);
+    if (apart && fits_x6s((int64_t)g.x * g.y * g.z, ext_a, ext_b, pbpl != nullptr, K8, N)) {
       const dim3 gs((unsigned)((N + 31) / 32), g.y, g.z);
       auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, gs, dim3(128), 0, L.stream, pa, pb, pc, (int)M, (int)N, (int)K, (int)lda, (int)ldb,

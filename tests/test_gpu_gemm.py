@@ -245,3 +245,27 @@ def test_few_tiles_give_the_large_kernel_bit_for_bit(gpu, name):
     np.testing.assert_array_equal(c0, c1[:M])
     if nw >= 0:
         np.testing.assert_array_equal(s0[:M // 128], s1[:M // 128])
+
+
+@pytest.mark.parametrize("over", ["A", "B"])
+@pytest.mark.parametrize("n", [33, 96, 128])
+def test_one_tile_product_over_its_operand(gpu, over, n):
+    """A product of one 128 x 128 tile whose result lies in an operand's cells
+    is the product with cells of its own, bit for bit."""
+    rng = np.random.default_rng(n)
+    a, b = (rng.standard_normal((n, n)).astype(np.float32) for _ in range(2))
+    bias = rng.standard_normal(n).astype(np.float32)
+    got = []
+    for shared in (False, True):
+        p = Program(max_frames=1)
+        c = {k: p.alloc(k, m) for k, m in (("a", n * n), ("b", n * n), ("c", n * n), ("bias", n))}
+        name = over.lower() if shared else "c"
+        out = c[name]
+        p.add(R.K_GEMM, [c["a"], c["b"], out, n, n, n, n, n, n, 0, 0, 1, c["bias"], -1, 0, 1, -1, -1, -1, 0, 1, -1])
+        print(f"case n={n} over {over if shared else None}", flush=True)
+        with R.HIPLazyRuntime(p, 0) as rt:
+            for k, v in (("a", a), ("b", b), ("bias", bias)):
+                rt.write(k, v)
+            rt.runNoCopy()
+            got.append(rt.read(name))
+    np.testing.assert_array_equal(got[1], got[0])
