@@ -163,7 +163,6 @@ static int colsum_chunks(int64_t rows, int nw = 0) {
   return (int)std::min<int64_t>(nw > 0 ? 2 * kColChunks : kColChunks, std::max<int64_t>(1, rows / 32));
 }
 
-// out_q (q < nw) rows of out0 (stride ld_out0) and the plain sum into plain_out.
 // Few rows: the two stages in one launch, a workgroup of 16 waves per 64
 // columns.  What stage 1's wave w of row chunk c sums is summed here by wave
 // (4c + w) % 16, and the sums are added in the stages' order, so the result is
@@ -220,6 +219,7 @@ __global__ __launch_bounds__(1024) void k_sum_one(const float* __restrict__ A, i
   }
 }
 
+// out_q (q < nw) rows of out0 (stride ld_out0) and the plain sum into plain_out.
 static int colsum_launch(const Launch& L, const float* A, int lda, const float* X, int nw, int rows, int cols,
                          float* ws, float* out0, int ld_out0, float* plain_out) {
   const int chunks = colsum_chunks(rows, nw);
@@ -254,7 +254,9 @@ int launch_colsum(const Launch& L, const dgen_hip_op& op) {
     DGEN_LAUNCH_CHECK("k_sum_one");
     return 0;
   }
-  if (rows <= kColOneRows && rows * cols <= kColOneCells) {
+  // (a sum over its own source waits for the whole first stage)
+  if (rows <= kColOneRows && rows * cols <= kColOneCells &&
+      written_apart({{out, cols}}, {{A, (rows - 1) * lda + cols}})) {
     hipLaunchKernelGGL(k_colsum_one, dim3((unsigned)((cols + 63) / 64)), dim3(1024), 0, L.stream, cell(L, A), (int)lda,
                        (int)rows, (int)cols, chunks, (int)((rows + chunks - 1) / chunks), cell(L, out));
     DGEN_LAUNCH_CHECK("k_colsum_one");

@@ -36,6 +36,22 @@ def test_one_launch_is_the_two_stage_sum(gpu, rows, cols):
     assert np.abs(two - ref).max() <= 32 * 6e-8 * np.abs(a).sum(0).max()
 
 
+@pytest.mark.parametrize("at", [0, 1, 70, 130 * 9 + 64])
+def test_sum_over_its_source(gpu, at):
+    """The result may lie in the summed matrix: the two stages read all of it
+    first, and so does a sum that takes one launch elsewhere."""
+    rows, cols = 40, 130
+    a = np.random.default_rng(at).standard_normal((rows, cols)).astype(np.float32)
+    p = Program(max_frames=1)
+    c, w = p.alloc("a", rows * cols), p.alloc("w", 256 * cols)
+    p.add(R.K_COLSUM, [c, c + at, rows, cols, cols, w])
+    print(f"case at={at}", flush=True)
+    with R.HIPLazyRuntime(p) as rt:
+        rt.write("a", a)
+        rt.runNoCopy()
+        np.testing.assert_array_equal(rt.read("a")[at:at + cols], colsum(a, cols))
+
+
 @pytest.mark.parametrize("rows", [1, 1023, 1024, 1025, 16384, 16385])
 def test_one_column(gpu, rows):
     a = np.random.default_rng(rows).standard_normal((rows, 1)).astype(np.float32)
