@@ -104,7 +104,9 @@ __device__ __forceinline__ float svf_step(const SvfK& K, float ks, float x, floa
   const float s2 = sat_div<SAT>(c2, ks);
   const float v3 = x - s2;
   const float v1 = K.a1 * s1 + K.a2 * v3;
-  // (doubling is exact, so the fma rounds as the product and difference do)
+  // (doubling is exact, so the fma rounds as the product and difference do;
+  // only past |v1| = 2^127, where the product would be infinite, a difference
+  // that is finite stays so)
   const float ic1 = __builtin_fmaf(2.0f, v1, -s1);
   const float v1p = (ic1 + s1) * 0.5f;
   const float v2 = s2 + K.g * v1p;

@@ -196,38 +196,53 @@ def test_saturating_training_loss_covers_a_ragged_last_chunk(B, T, chunk):
     assert np.linalg.norm(g - g64) <= 1e-4 * np.linalg.norm(g64)
 
 
-@pytest.mark.parametrize("B,T,chunk,signal", [(1, 257, 256, "noise"), (3, 5000, 256, "noise"), (64, 4096, 256, "noise"),
-                                              (70, 3001, 7, "noise"), (256, 20000, 512, "noise"),
-                                              (300, 6145, 96, "noise"), (66, 16384, 256, "click"),
-                                              (5, 12000, 256, "nan"), (64, 9000, 100, "inf")])
-def test_saturating_spans_equal_the_frame_loop(B, T, chunk, signal):
-    """The saturating forward as spans run side by side leaves y, the cells
-    and the loss partials of the per-lane frame loop bit for bit: ragged lane
-    groups, spans and chunks; a click after which the states shrink together
-    and never meet (the repair's part); non-finite input from some frame on."""
+def span_inputs(B, T, signal):
     cfg = SvfConfig(B=B, T=T, saturating=True)
     rng = np.random.default_rng(B + T)
     x = rng.uniform(-1, 1, (T, B)).astype(np.float32)
-    if signal == "click":
+    if "click" in signal:
         x[1000:] = 0.0
-    elif signal in ("nan", "inf"):
-        x[T // 3, ::2] = np.nan if signal == "nan" else np.inf
+    elif "noise" not in signal:
+        x[T // 3, ::2] = np.nan if "nan" in signal else np.inf
     tgt = rng.uniform(-1, 1, (T, B)).astype(np.float32)
     prm = cfg.params().reshape(3, B).copy()
     prm[2, ::3] *= 0.01  # lanes that hardly saturate forget most slowly
-    print(f"case B={B} T={T} chunk={chunk} {signal}", flush=True)
+    return cfg, dict(x=x, target=tgt, mod=cfg.modulation(), env=cfg.envelope(), params=prm)
+
+
+@pytest.mark.parametrize("train", [True, False], ids=["train", "render"])
+@pytest.mark.parametrize("B,T,chunk,signal", [(1, 257, 256, "noise"), (3, 5000, 256, "noise"),
+                                              (64, 4096, 256, "noise"), (70, 3001, 48, "noise"),
+                                              (256, 20000, 512, "noise"), (300, 6145, 96, "noise"),
+                                              (66, 16384, 256, "click"), (5, 12000, 256, "nan"),
+                                              (65, 9000, 112, "inf"), (1, 17, 16, "noise"),
+                                              (70, 3001, 7, "noise, loop"), (64, 9000, 100, "inf, loop"),
+                                              (1, 256, 256, "noise, loop")])
+def test_saturating_spans_equal_the_frame_loop(B, T, chunk, signal, train):
+    """The saturating forward as spans run side by side leaves y, the cells
+    and the loss partials of the per-lane frame loop bit for bit, in training
+    and rendering: ragged lane groups, spans and chunks; a click after which
+    the states shrink together and never meet (the repair's part); non-finite
+    input from some frame on.  "loop": chunks that are no whole groups of 16
+    frames, or one chunk alone, run the frame loop either way."""
+    cfg, inputs = span_inputs(B, T, signal)
+    print(f"case B={B} T={T} chunk={chunk} {signal} train={train}", flush=True)
     got = {}
     for spans in (0, 1):
-        prog = svf_program(cfg, optimizer=False, chunk=chunk)
-        assert prog.ops[0].kernel == R.K_SVF_SEQ and prog.ops[0].arg[15] == 1
-        prog.ops[0].arg[15] = spans
+        prog = svf_program(cfg, train=train, optimizer=False, chunk=chunk)
+        op = prog.ops[0]
+        assert op.kernel == R.K_SVF_SEQ and op.arg[15] == 1
+        op.arg[15] = spans
+        op.arg[14] = prog.alloc("own_span_states", 6 * -(-T // chunk) * B)
         with HIPLazyRuntime(prog) as rt:
-            for name, a in (("x", x), ("target", tgt), ("mod", cfg.modulation()), ("env", cfg.envelope()),
-                            ("params", prm)):
-                rt.write(name, a)
+            for name, a in inputs.items():
+                if name in prog.cells:
+                    rt.write(name, a)
             for _ in range(2):
                 rt.runNoCopy()
-            got[spans] = [rt.read(n) for n in ("y", "cells", "loss_partials")]
+            got[spans] = [rt.read(n) for n in (("y", "cells", "loss_partials") if train else ("y",))]
+            # the spans leave their states behind, the loop nothing
+            assert rt.read("own_span_states").any() == (spans == 1 and "loop" not in signal)
     for a, b in zip(got[0], got[1]):
         bits = [np.where(np.isnan(v), 0, v.view(np.uint32)) for v in (a, b)]  # a NaN's sign is not defined
         np.testing.assert_array_equal(np.isnan(a), np.isnan(b))
