@@ -50,6 +50,8 @@ struct StftArgs {
   float* gpart;        // [S][nblk][N/2 + 1] (backward)
   int S, T, H, ntiles, nblk, tile, rounds;
   int logv;            // windows 2^logv hops apart do not overlap (forward)
+  unsigned hmul;       // n / H = n hmul >> hshift for 0 <= n < 2^30 (forward)
+  int hshift;
   float invT;
 };
 
@@ -121,8 +123,9 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
   for (int i = tid; i <= M; i += kThreads) gain[i] = a.gains[i];
   for (int i = tid; i < ((a.tile + 63) & ~63); i += kThreads) acc[i] = 0.0f;
   // windows h = w*H with outputs [h, h+N) meeting [a0, a1)
-  const int w_lo = a0 - N < 0 ? 0 : (a0 - N) / H + 1;
-  const int w_hi = (a1 - 1) / H;
+  auto hops = [&](int n) { return (int)(((uint64_t)(unsigned)n * a.hmul) >> a.hshift); };  // n / H
+  const int w_lo = a0 - N < 0 ? 0 : hops(a0 - N) + 1;
+  const int w_hi = hops(a1 - 1);
   const SwzBuf buf(lbuf, slot * M);
   const int sj = buf.part(j);
   const HwRegTwiddle<LOGM> tw(j);
@@ -204,7 +207,7 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
   };
   __syncthreads();
   int q = residue(slot), w = window(slot, q);
-  int u = residue(0), end = before(u + 1);  // slot 0's residue, and its windows' end
+  int u = blocks == 1 ? rl : 0, end = before(u + 1);  // slot 0's residue, and its windows' end
   fetch(w);
   for (int k0 = 0; k0 < nw; k0 += W) {
     c2 v[8];
@@ -267,7 +270,8 @@ __global__ __launch_bounds__(kThreads) void k_stft_fwd(StftArgs a) {
       lds_barrier();
       more = end < kn;
       if (end <= kn && end < nw) {
-        u = residue(end);
+        ++u;
+        if (before(u + 1) == end) u = rl;  // only residues between rh and rl have no windows
         end = before(u + 1);
       }
     }
@@ -471,6 +475,10 @@ int launch_stft_fwd(const Launch& L, const dgen_hip_op& op) {
   a.ntiles = (int)ntiles;
   a.tile = (int)tile;
   while ((H << a.logv) < N) ++a.logv;
+  // (hmul H exceeds 2^hshift by less than H <= 2^(hshift - 30))
+  a.hshift = 30;
+  while ((1ll << (a.hshift - 30)) < H) ++a.hshift;
+  a.hmul = (unsigned)(((1ll << a.hshift) + H - 1) / H);
   a.invT = 1.0f / (float)T;
   hipLaunchKernelGGL(fwd_kernel(logn), dim3((unsigned)ntiles, (unsigned)S), dim3(kThreads),
                      (unsigned)((tile + 63) / 64 * 64 * sizeof(float)), L.stream, a);
