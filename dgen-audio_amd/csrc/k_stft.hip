@@ -305,8 +305,8 @@ struct BwdLds {
   c2 aux[2048];
 };
 
-// (held to four waves per SIMD up to N = 1024: 53 -> 46 us at 8 x 2^20, N = 1024;
-// at 2048 that spills)
+// (held to four waves per SIMD up to N = 1024, for 3 spilled registers at N =
+// 512 and one at 1024: 53 -> 46 us at 8 x 2^20, N = 1024; at 2048 far more spill)
 template <int LOGN>
 __global__ __launch_bounds__(kThreads, LOGN <= 10 ? 4 : 2) void k_stft_bwd(StftArgs a) {
   constexpr int N = 1 << LOGN, M = N / 2, LOGM = LOGN - 1, P = M / 8, W = kThreads / P;

@@ -630,8 +630,9 @@ def svf_program(cfg: SvfConfig, train: bool = True, optimizer: bool = True, satu
     and res[k] (and, saturating, kSat[k]).
 
     Linear (kSat the constant 0): the forward is a chunked scan (fp64 chunk
-    maps, per-lane carry composition, fp32 replay).  Saturating: one lane per
-    thread over all frames.  ``train=False`` renders y only.  With
+    maps, per-lane carry composition, fp32 replay).  Saturating: spans of
+    frames side by side, run again until each starts where the one before
+    ends (the frame loop's bits).  ``train=False`` renders y only.  With
     ``train=True``: forward storing the cells entering every frame, loss
     sum (y - target)^2, BPTT to the parameters as a chunked reverse scan
     (``xbar``: also d loss / d x), and (``optimizer``) one Adam step.  With
@@ -856,9 +857,9 @@ def stft_tile(S: int, T: int, N: int, H: int) -> int:
     than 512) while that makes at most STFT_GROUPS workgroups.  A tile runs its
     windows a few at a time, so a short signal wants short tiles on more of
     the chip; a long one wants long tiles, whose edges repeat fewer windows.
-    (2 x 44101 samples, N = 512: 36 us at 8192, 7.5 at 512; 4 x 200000, N =
-    2048: 49 at 8192, 25 at 2048, 38 at 1024; 8 x 2^20, N = 1024: 86 at 8192, 96
-    at 4096.)"""
+    (2 x 44101 samples, N = 512: 35 us at 8192, 11 at 1024, 8 at 512; 1 x 2^20,
+    N = 2048: 54 at 8192, 32 at 2048, 44 at 1024; 8 x 2^20, N = 1024: 85 at 8192,
+    84 at 4096; N = 2048: 115 and 138.)  y does not depend on it."""
     tile = STFT_TILE
     while tile > 512 and S * ((T + tile // 2 - 1) // (tile // 2)) <= STFT_GROUPS:
         tile //= 2
